@@ -1,20 +1,13 @@
 // backward.hip — rasterize backward and project backward for gfx950.
 //
-// rasterize_backward: one single-wave workgroup per 8x8 pixel block of a
-// 16x16 tile, one pixel per lane.  Every pixel replays the tile's splats front
-// to back with the same per-pair arithmetic as the reference's replay
+// rasterize_backward: every pixel walks its tile's splats front to back with
+// the per-pair arithmetic of the reference's replay
 // (crates/brush-render-bwd/src/kernels/rasterize_backwards.rs:79-443, where
 // instead a 32-lane workgroup owns 32 splats and walks the pixels on a
 // diagonal); the transmittance / remaining-colour state never leaves the
-// lane's registers.  Each wave stages the tile's splats in LDS in batches of
-// 64 and keeps those that may touch its block (a ballot of a conservative
-// rectangle test), so the four blocks of a tile run independently, without
-// workgroup barriers, and a block whose 64 pixels have all saturated stops.
-// For a splat with any contributing pixel the wave sums its 9-11 gradient
-// lanes over all 64 pixels with a transposed reduction (permlane32 and
-// permlane16 swaps fold four lanes into one register, then four DPP row
-// steps), which leaves up to four different gradient lanes in lanes 15, 31,
-// 47 and 63, so one float-atomic instruction adds four of them.
+// lane's registers, and a splat's gradient sums leave the workgroup as one
+// float atomic per value.  The fused backward reads which pairs contributed
+// from the forward's record; rasterize_backward on its own decides it again.
 //
 // project_backward: one thread per *global* id, so every dense output row is
 // written exactly once (zeros for culled splats or splats without gradient)
@@ -30,28 +23,13 @@
 #include "bh_splat_record.h"
 #include "bh_tile_walk.h"
 
-// Candidates staged per batch by the recorded backward (32 or 64).  32
-// keeps its LDS at 9 KB (17 workgroups per CU) with three summing slots.
-#ifndef BH_BWD_BATCH
-#define BH_BWD_BATCH 32
-#endif
-
 namespace bh {
 
-// Sum of x over each 16-lane row of the wave, left in the row's last lane
-// (inclusive Hillis-Steele steps as DPP adds).
+// x plus the x of the lane DPP control CTRL names.
 template <int CTRL>
 __device__ __forceinline__ float dpp_add(float x) {
     return x + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(x), CTRL, 0xF, 0xF, true));
 }
-__device__ __forceinline__ float row_sum_last_lane(float x) {
-    x = dpp_add<0x111>(x);  // row_shr:1
-    x = dpp_add<0x112>(x);  // row_shr:2
-    x = dpp_add<0x114>(x);  // row_shr:4
-    x = dpp_add<0x118>(x);  // row_shr:8
-    return x;
-}
-
 // Transposed wave reduction.  psum32(a, b): rows 0-1 (lanes 0-31) hold a
 // summed over lanes i and i + 32, rows 2-3 hold b likewise.  psum16(p, q) of
 // two such values: row 0 holds p's rows 0+1, row 1 q's rows 0+1, row 2 p's
@@ -66,6 +44,12 @@ __device__ __forceinline__ float psum16(float p, float q) {
     return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
+// Candidates staged per batch by the recorded backward (32 or 64).  32
+// keeps its LDS at 9 KB (17 workgroups per CU) with three summing slots.
+#ifndef BH_BWD_BATCH
+#define BH_BWD_BATCH 32
+#endif
+
 constexpr int kNG = 11;
 
 // One workgroup (a single wave) per 8x8 pixel block of a 16x16 tile.  The
@@ -77,241 +61,6 @@ __device__ __forceinline__ void block_of_workgroup(uint32_t g, uint32_t& tile, u
     const uint32_t slot = g >> 3;
     tile = ((slot / BPT) << 3) | (g & 7u);
     blk = slot % BPT;
-}
-
-template <bool SMOOTH, bool REFINE, bool DEPTH, int TH>
-__global__ __launch_bounds__(64) void rasterize_backward_kernel(
-    uint32_t img_w, uint32_t img_h, uint32_t tile_bw, uint32_t num_tiles, float bg_r, float bg_g, float bg_b,
-    uint32_t num_visible, const float* __restrict__ out_img, const float* __restrict__ projected,
-    const uint32_t* __restrict__ cgids, const uint32_t* __restrict__ offsets, const float* __restrict__ v_output,
-    const uint32_t* __restrict__ row_of, const uint32_t* __restrict__ order, float* __restrict__ v_combined) {
-    constexpr uint32_t CH = DEPTH ? 5u : 4u;
-    __shared__ float4 s_xyco[64];  // x, y, conic c00, c01
-    __shared__ float4 s_crgb[64];  // conic c11, opacity, r, g (staged_colour)
-    __shared__ float4 s_bd[64];    // b (staged_colour), depth, sigma cutoff
-    __shared__ uint32_t s_cid[64];
-
-    uint32_t tile, blk;
-    block_of_workgroup<TH>(blockIdx.x, tile, blk);
-    if (tile >= num_tiles) return;
-    if (order) tile = order[tile];
-    const uint32_t lane = threadIdx.x;
-    const uint32_t ox = (tile % tile_bw) * 16u + (blk & 1u) * 8u;
-    const uint32_t oy = (tile / tile_bw) * (uint32_t)TH + (blk >> 1) * 8u;
-    const uint32_t px = ox + (lane & 7u), py = oy + (lane >> 3);
-    const bool inside = px < img_w && py < img_h;
-    const float pcx = (float)px + 0.5f, pcy = (float)py + 0.5f;
-
-    // Pixel state of the front-to-back replay (rasterize_backwards.rs:193-250):
-    // remaining colour (final minus background pre-roll) and transmittance.
-    float sx = 0.0f, sy = 0.0f, sz = 0.0f, sw = 0.0f, sd = 0.0f;
-    float vox = 0.0f, voy = 0.0f, voz = 0.0f, vow = 0.0f, vod = 0.0f, final_a = 0.0f;
-    if (inside) {
-        const size_t pix = (size_t)py * img_w + px;
-        const float* o = out_img + pix * CH;
-        const float* vo = v_output + pix * CH;
-        final_a = o[3];
-        const float t_final = 1.0f - final_a;
-        sx = o[0] - t_final * bg_r;
-        sy = o[1] - t_final * bg_g;
-        sz = o[2] - t_final * bg_b;
-        sw = 1.0f;
-        vox = vo[0];
-        voy = vo[1];
-        voz = vo[2];
-        vow = (vo[3] - (bg_r * vox + bg_g * voy + bg_b * voz)) * t_final;
-        if (DEPTH) {
-            sd = o[4];
-            vod = vo[4];
-        }
-    }
-    const uint32_t lo = offsets[2 * tile], hi = offsets[2 * tile + 1];
-    // Work is concentrated in few tiles (at config 1, 28 % of the tiles hold
-    // splats; the heaviest replays ~480, the mean ~53), so the kernel ends
-    // with the long blocks sharing their SIMDs.  A block's wave priority
-    // rises with its tile's splat count, so the SIMD issues long blocks first.
-    const uint32_t len = hi - lo;
-    if (len >= 256u)
-        __builtin_amdgcn_s_setprio(3);
-    else if (len >= 128u)
-        __builtin_amdgcn_s_setprio(2);
-    else if (len >= 64u)
-        __builtin_amdgcn_s_setprio(1);
-    const float img_wf = (float)img_w, img_hf = (float)img_h;
-    const float inv_final_a = __builtin_amdgcn_rcpf(bh_maxf(final_a, 1.0e-5f));
-    const float bx0 = (float)ox + 0.5f, by0 = (float)oy + 0.5f;
-    bool wave_live = __ballot(sw > 1.0e-4f) != 0ull;
-
-    for (uint32_t b = lo; wave_live && b < hi; b += 64u) {
-        const uint32_t cnt = min(64u, hi - b);
-        bool touch = false;
-        if (lane < cnt) {
-            const uint32_t c = min(cgids[b + lane], num_visible - 1u);
-            const float2* prow = reinterpret_cast<const float2*>(projected + (size_t)c * 10);
-            const float2 r0 = prow[0], r1 = prow[1], r2 = prow[2], r3 = prow[3], r4 = prow[4];
-            const float cut = sigma_cutoff<SMOOTH>(r2.y);
-            s_xyco[lane] = make_float4(r0.x, r0.y, r1.x, r1.y);
-            s_crgb[lane] = make_float4(r2.x, r2.y, staged_colour(r3.x), staged_colour(r3.y));
-            // the cutoff on the power in base 2 (power log2(e); the cutoff's
-            // margin of 1e-3 covers the rounding)
-            s_bd[lane] = make_float4(staged_colour(r4.x), r4.y, kLog2e * cut, 0.0f);
-            s_cid[lane] = row_of ? row_of[c] : c;
-            touch = may_touch_rect(r0.x, r0.y, S2{r1.x, r1.y, r2.x}, cut, bx0, by0, bx0 + 7.0f, by0 + 7.0f);
-        }
-        // splats of the batch that may touch this block, in order
-        uint64_t todo = __ballot(touch);
-        wave_lds_fence();
-        while (todo) {
-            const uint32_t j = (uint32_t)__builtin_ctzll(todo);
-            todo &= todo - 1ull;
-            const float4 xc = s_xyco[j];
-            const float4 cr4 = s_crgb[j];
-            const float4 bd = s_bd[j];
-            const S2 conic{xc.z, xc.w, cr4.x};
-            const float opac = cr4.y;
-            const float dx = xc.x - pcx, dy = xc.y - pcy;
-            // the forward's Gaussian (bh_math.h: the power in base 2)
-            float ka, kb, kc;
-            bh_conic_log2(conic.c00, conic.c01, conic.c11, &ka, &kb, &kc);
-            const float power = bh_power_log2(ka, kb, kc, dx, dy);
-            const bool maybe = sw > 1.0e-4f && power >= 0.0f && !(power > bd.z);
-            if (__ballot(maybe) == 0ull) continue;
-            // lanes outside `maybe` compute values that the selects below discard
-            const float gaussian = bh_exp2_neg(-power);
-            const float alpha = bh_minf(0.999f, opac * gaussian);
-            const float w = SMOOTH ? cutoff_weight(alpha) : (alpha >= kCutMid ? 1.0f : 0.0f);
-            const bool pass = maybe && w > 0.0f;
-            const float ae = SMOOTH ? alpha * w : (alpha >= kCutMid ? alpha : 0.0f);
-            const float next_t = sw * (1.0f - ae);
-            const bool saturate = pass && next_t <= 1.0e-4f;
-            const bool contrib = pass && !saturate;
-            if (saturate) sw = 0.0f;
-            if (__ballot(contrib) == 0ull) {
-                wave_live = __ballot(sw > 1.0e-4f) != 0ull;
-                if (!wave_live) break;
-                continue;
-            }
-            float g[12];
-            {
-#pragma clang fp contract(fast)
-                // Gradient-only arithmetic and the remaining-colour state, which
-                // feeds only gradients: products and sums fuse into FMAs here.
-                // The replay's decisions above (alpha, transmittance, saturation)
-                // stay uncontracted, bit for bit the forward's.
-                // staged colours: max(c, 0) in value, the c >= 0 gate in the sign bit
-                const float cr = cr4.z, cgc = cr4.w, cb = bd.x;
-                const float vis = ae * sw;
-                g[5] = contrib && colour_gate(cr) ? vis * vox : 0.0f;
-                g[6] = contrib && colour_gate(cgc) ? vis * voy : 0.0f;
-                g[7] = contrib && colour_gate(cb) ? vis * voz : 0.0f;
-                // gradient-only quantities: hardware reciprocal / sqrt (1 ulp)
-                const float ra = __builtin_amdgcn_rcpf(1.0f - ae);
-                const float dot_rgb = ((sw * cr - sx) * vox + (sw * cgc - sy) * voy + (sw * cb - sz) * voz) * ra;
-                const float v_ae = dot_rgb + vow * ra;
-                // with the hard cutoff the weight is a step and its derivative 0.
-                // The position, conic, opacity and refine lanes are gated on
-                // contributing and unclamped (o G <= 0.999) pairs.  Lanes outside
-                // `maybe` may hold any alpha and gaussian: a sigma far below zero
-                // (rounding on a nearly singular conic) overflows the exponential's
-                // range reduction into inf or a negative value.  So the selects sit
-                // on v_sigma and on the opacity lane; a zero v_sigma then zeroes the
-                // position, conic and refine lanes (up to the sign of a zero), whose
-                // other factors dx, dy and the conic (|c| <= 10: every 2D covariance
-                // carries a blur of at least 0.1 on its diagonal) are finite.
-                const bool unclamped = opac * gaussian <= 0.999f;
-                const bool gate = contrib && unclamped;
-                const float v_alpha = SMOOTH ? v_ae * (w + alpha * cutoff_weight_deriv(alpha)) : v_ae * w;
-                const float v_sigma = gate ? -alpha * v_alpha : 0.0f;
-                const float vxy_x = v_sigma * (conic.c00 * dx + conic.c01 * dy);
-                const float vxy_y = v_sigma * (conic.c01 * dx + conic.c11 * dy);
-                g[2] = 0.5f * v_sigma * dx * dx;
-                g[3] = v_sigma * dx * dy;
-                g[4] = 0.5f * v_sigma * dy * dy;
-                g[0] = vxy_x;
-                g[1] = vxy_y;
-                g[8] = gate ? v_alpha * gaussian : 0.0f;
-                g[9] = REFINE ? __builtin_amdgcn_sqrtf(vxy_x * img_wf * vxy_x * img_wf + vxy_y * img_hf * vxy_y * img_hf) *
-                                    inv_final_a
-                              : 0.0f;
-                g[10] = DEPTH && contrib ? vis * vod : 0.0f;
-                g[11] = 0.0f;
-                if (contrib) {
-                    sx = sx - vis * cr;
-                    sy = sy - vis * cgc;
-                    sz = sz - vis * cb;
-                    if (DEPTH) sd = sd - vis * bd.y;
-                }
-            }
-            if (contrib) sw = next_t;
-            // whole-wave sums: rows of q0 hold lanes 0, 2, 1, 3; of q1 lanes 4, 6,
-            // 5, 7; of q2 lanes 8, 10, 9, 11 (8, 8, 9, 9 without depth, of which
-            // one lane each is added: two lanes of one atomic instruction on one
-            // address measured 124 us per frame slower)
-            const float q0 = row_sum_last_lane(psum16(psum32(g[0], g[1]), psum32(g[2], g[3])));
-            const float q1 = row_sum_last_lane(psum16(psum32(g[4], g[5]), psum32(g[6], g[7])));
-            const float p4 = psum32(g[8], g[9]);
-            const float q2 = row_sum_last_lane(DEPTH ? psum16(p4, psum32(g[10], g[11])) : psum16(p4, p4));
-            // the splat's gradient row: wave-uniform, so its address is scalar
-            const uint32_t cid = __builtin_amdgcn_readfirstlane(s_cid[j]);
-            float* dst = v_combined + (size_t)cid * kNG;
-            // one atomic instruction for all three sums: q1's and q2's row totals
-            // move from lane 15 of each row to lanes 14 and 13 (DPP row_shl),
-            // so lanes 13-15 of a row add to three distinct words of the row
-            const float q1s = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q1), 0x101, 0xF, 0xF, true));
-            const float q2s = __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(q2), 0x102, 0xF, 0xF, true));
-            const uint32_t r = lane & 15u;
-            if (r >= 13u) {
-                const uint32_t row = lane >> 4;
-                const uint32_t k = (row & 1u) * 2u + (row >> 1);
-                const bool want = DEPTH ? (k == 0u || (k == 1u && REFINE) || k == 2u) : (k == 0u || (row == 2u && REFINE));
-                const uint32_t off = r == 15u ? k : r == 14u ? 4u + k : (DEPTH ? 8u + k : 8u + (row >> 1));
-                const float val = r == 15u ? q0 : r == 14u ? q1s : q2s;
-                if (r != 13u || want) unsafeAtomicAdd(dst + off, val);
-            }
-            wave_live = __ballot(sw > 1.0e-4f) != 0ull;
-            if (!wave_live) break;
-        }
-        wave_lds_fence();
-    }
-}
-
-void launch_rasterize_backward(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile_bw, uint32_t tile_bh,
-                               const float* bg, uint32_t num_visible, const float* out_img, const float* projected, const uint32_t* cgids,
-                               const uint32_t* offsets, const float* v_output, uint32_t flags,
-                               const uint32_t* row_of, const uint32_t* order, float* v_combined) {
-    const uint32_t num_tiles = tile_bw * tile_bh;
-    if (num_tiles == 0 || num_visible == 0) return;
-    const bool smooth = (flags & BH_FLAG_SMOOTH_CUTOFF) != 0;
-    const bool refine = (flags & BH_FLAG_REFINE_WEIGHT) != 0;
-    const bool depth = (flags & BH_FLAG_RENDER_DEPTH) != 0;
-    const bool fine = (flags & BH_FLAG_TILE_16X8) != 0;
-    const uint32_t groups = div_up(num_tiles, 8) * (fine ? 16u : 32u);
-    KernelTimer t(ctx, "rasterize_backward");
-#define BH_RB_T(S, R, D, T)                                                                                      \
-    launch(ctx, rasterize_backward_kernel<S, R, D, T>, dim3(groups), dim3(64), 0u, img_w, img_h, tile_bw, num_tiles,   \
-           bg[0], bg[1], bg[2], num_visible, out_img, projected, cgids, offsets, v_output, row_of, order, v_combined)
-#define BH_RB(S, R, D) \
-    do {               \
-        if (fine)      \
-            BH_RB_T(S, R, D, 8); \
-        else           \
-            BH_RB_T(S, R, D, 16); \
-    } while (0)
-    if (smooth) {
-        if (refine) {
-            if (depth) BH_RB(true, true, true); else BH_RB(true, true, false);
-        } else {
-            if (depth) BH_RB(true, false, true); else BH_RB(true, false, false);
-        }
-    } else {
-        if (refine) {
-            if (depth) BH_RB(false, true, true); else BH_RB(false, true, false);
-        } else {
-            if (depth) BH_RB(false, false, true); else BH_RB(false, false, false);
-        }
-    }
-#undef BH_RB_T
-#undef BH_RB
 }
 
 // ---- fused rasterize backward from the forward's record ----------------------------
@@ -422,7 +171,8 @@ __global__ __launch_bounds__(64) void rasterize_backward_recorded_kernel(
     const uint32_t lane = threadIdx.x;
     const uint32_t ox = (tile % tile_bw) * 16u + (blk & 1u) * 8u;
     const uint32_t oy = (tile / tile_bw) * (uint32_t)TH + (blk >> 1) * 8u;
-    const uint32_t px = ox + (lane & 7u), py = oy + (lane >> 3);
+    // lane 16 s + p: pixel p of 4x4 sub-block s (the record's bit order)
+    const uint32_t px = ox + ((lane >> 4) & 1u) * 4u + (lane & 3u), py = oy + (lane >> 5) * 4u + ((lane >> 2) & 3u);
     const bool inside = px < img_w && py < img_h;
     const float pcx = (float)px + 0.5f, pcy = (float)py + 0.5f;
 
@@ -447,7 +197,8 @@ __global__ __launch_bounds__(64) void rasterize_backward_recorded_kernel(
         if (DEPTH) vod = vo[4];
         dsum = sx * vox + sy * voy + sz * voz;
     }
-    // long blocks first (work sits in few tiles; see the replay kernel above)
+    // long blocks first: work is concentrated in few tiles, and a frame ends
+    // with the long blocks sharing their SIMDs
     const uint32_t len = end - lo;
     if (len >= 256u)
         __builtin_amdgcn_s_setprio(3);
@@ -709,6 +460,473 @@ __global__ __launch_bounds__(64) void rasterize_backward_recorded_kernel(
     }
 }
 
+// A workgroup of four waves owns an 8x8 block, each wave a 4x4 sub-block as in
+// the forward blend: lane 4 p + k holds pixel p and the k-th of the four
+// candidates a step takes.  The pair's gradient terms are evaluated once, by
+// its own lane; the transmittance and D run over the four candidates in every
+// lane of the pixel's quad (DPP broadcasts).  A candidate's K sums over the
+// sixteen pixels are folded four at a time over the lanes' upper bits
+// (permlane swaps) and added along the rows, so that one LDS store of the wave
+// puts all sums of the step in the candidates' rows, one row per sub-block;
+// the rows leave the workgroup once per batch, with the splat's factors, as
+// one float atomic per value.
+//
+// With REPLAY it is rasterize_backward's kernel instead: no record, so a
+// candidate is staged where it may touch the sub-block, and which pairs
+// contributed is decided as the forward decides it (candidates [lo, hi) of
+// `off`, rows of v_rows by row_of or by compact id).
+//
+// What bounds it: below a few thousand blocks the chip is not full, and a
+// block's time is the issue of its own instructions (a wave retires one every
+// five to nine cycles): one wave per 8x8 block, a candidate at a time, took
+// ~300 ns a candidate.  A step here is ~105 VALU for four candidates of a
+// quarter of the pixels.  Rasterize backward from the record, one wave per
+// block -> four: 256x256, 100k splats 157 -> 58 us; 640x480 (4,800 blocks)
+// 93 -> 51 us, 129 -> 59 us where the splats crowd, 131 -> 123 us where every
+// tile is loaded alike; 800x600 (7,600) 93 -> 64, 126 -> 75, 225 -> 235 us;
+// 1024x768 (12,288) 85 -> 82, 107 -> 96, 279 -> 335 us: a full chip issues 1.4
+// times the instructions.  The replay was slower at every size as one wave per
+// block (256x256 266 -> 81, 640x360 167 -> 57, 800x600 165 -> 81, 1280x720
+// 215 -> 128 us; every tile loaded alike at 1280x720 465 -> 408 us).  (The sums as 16x4 by 4x16 matrix products on the
+// MFMA units were slower, ten dependent products a step; so were LDS float
+// atomics into one row per candidate, ~140 LDS cycles a step.)
+template <bool REPLAY, bool SMOOTH, bool REFINE, bool DEPTH, int TH>
+__global__ __launch_bounds__(256) void rasterize_backward_quad_kernel(
+    uint32_t img_w, uint32_t img_h, uint32_t tile_bw, uint32_t num_tiles, float bg_r, float bg_g, float bg_b,
+    uint32_t num_visible, const float* __restrict__ out_img, const float* __restrict__ projected,
+    const uint32_t* __restrict__ cgids, const uint32_t* __restrict__ off, SplatRecord rec,
+    const float* __restrict__ v_output, const uint32_t* __restrict__ row_of, const uint32_t* __restrict__ order,
+    float* __restrict__ v_rows, FillRanges fill, uint32_t fill_slots, uint32_t all_slots) {
+    constexpr uint32_t CH = DEPTH ? 5u : 4u;
+    constexpr uint32_t BPT = 2u * (uint32_t)TH / 8u;
+    // sums per splat: v_sigma dx, v_sigma dy, v_sigma dx dx, v_sigma dx dy,
+    // v_sigma dy dy, vis v_r, vis v_g, vis v_b, the opacity lane, (refine), (depth)
+    constexpr int K = 9 + (REFINE ? 1 : 0) + (DEPTH ? 1 : 0);
+    constexpr uint32_t NB = 128;     // candidates per batch
+    constexpr uint32_t GS = 12;      // floats per row of sums
+    // the conic from its scaled form (bh_conic_log2): c00 = 2 ln2 a,
+    // c01 = ln2 b, c11 = 2 ln2 c
+    constexpr float kLn2 = 0.69314718055994530942f;
+    constexpr float kTwoLn2 = 1.38629436111989061883f;
+    // slot NB pads a step of fewer than four candidates (no pixel contributes)
+    __shared__ float4 s_geo[NB + 1];  // x, y, scaled conic a, b (bh_conic_log2)
+    __shared__ float4 s_op[NB + 1];   // scaled conic c, opacity, max(r, 0), max(g, 0)
+    // max(b, 0) and, with REPLAY, the cutoff on the power in base 2 (bits), the
+    // colour gates (bit c where channel c >= 0), the gradient row
+    __shared__ uint4 s_aux[NB + 1];
+    // contributing pixels (bh_splat_record.h); with REPLAY bit 16 s where the
+    // candidate may touch sub-block s
+    __shared__ unsigned long long s_mask[NB + 1];
+    __shared__ float s_sum[4][(NB + 1) * GS];  // [sub-block][candidate][value]
+    __shared__ float s_dump[64];         // where lanes without a value store
+    __shared__ unsigned long long s_touch[5][2];  // [sub-block; any][staging wave]
+    __shared__ uint16_t s_list[4][NB + 16];       // each sub-block's candidates
+    __shared__ uint16_t s_any[NB];                // the block's
+    __shared__ uint32_t s_alive[4];
+
+    // fill_slots of the all_slots slots of 8 workgroups (one per XCD) zero
+    // the fill ranges, spread evenly among the blend's: slot s is a fill
+    // slot where floor((s + 1) F / T) > floor(s F / T), the fill slot
+    // floor(s F / T), else blend slot s - floor(s F / T)
+    const uint32_t t = threadIdx.x;
+    uint32_t g = blockIdx.x;
+    if (fill_slots) {
+        const uint32_t s = g >> 3;
+        const uint32_t f0 = (uint32_t)((uint64_t)s * fill_slots / all_slots);
+        const uint32_t f1 = (uint32_t)((uint64_t)(s + 1u) * fill_slots / all_slots);
+        if (f1 > f0) {
+            fill_ranges_strided<true>(fill, (uint64_t)(f0 * 8u + (g & 7u)) * 256u + t, (uint64_t)fill_slots * 2048u);
+            return;
+        }
+        g = ((s - f0) << 3) | (g & 7u);
+    }
+    uint32_t tile, blk;
+    block_of_workgroup<TH>(g, tile, blk);
+    if (tile >= num_tiles) return;
+    if (order)
+        tile = order[tile];
+    else if (!REPLAY && rec.order.list) {
+        // the order the forward blend recorded (tiles some pixel blended)
+        tile = ordered_tile(tile, rec.order.count, rec.order.list, num_tiles);
+        if (tile >= num_tiles) return;
+    }
+    const uint32_t lo = off[2 * tile], hi = off[2 * tile + 1];
+    const uint32_t end = REPLAY ? hi : rec.block_end[tile * BPT + blk];
+    if (end <= lo) return;
+    const uint32_t lane = t & 63u, sub = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t >> 6));
+    const uint32_t slot = lane & 3u, p = lane >> 2;
+    const uint32_t px = (tile % tile_bw) * 16u + (blk & 1u) * 8u + (sub & 1u) * 4u + (p & 3u);
+    const uint32_t py = (tile / tile_bw) * (uint32_t)TH + (blk >> 1) * 8u + (sub >> 1) * 4u + (p >> 2);
+    const bool inside = px < img_w && py < img_h;
+    const float pcx = (float)px + 0.5f, pcy = (float)py + 0.5f;
+
+    // transmittance and D = (final colour minus background pre-roll) . v_out
+    // (rasterize_backwards.rs:193-250)
+    float sw = 0.0f, dsum = 0.0f;
+    float vox = 0.0f, voy = 0.0f, voz = 0.0f, vow = 0.0f, vod = 0.0f, final_a = 0.0f;
+    if (inside) {
+        const size_t pix = (size_t)py * img_w + px;
+        const float* o = out_img + pix * CH;
+        const float* vo = v_output + pix * CH;
+        final_a = o[3];
+        const float t_final = 1.0f - final_a;
+        const float sx = o[0] - t_final * bg_r;
+        const float sy = o[1] - t_final * bg_g;
+        const float sz = o[2] - t_final * bg_b;
+        sw = 1.0f;
+        vox = vo[0];
+        voy = vo[1];
+        voz = vo[2];
+        vow = (vo[3] - (bg_r * vox + bg_g * voy + bg_b * voz)) * t_final;
+        if (DEPTH) vod = vo[4];
+        dsum = sx * vox + sy * voy + sz * voz;
+    }
+    // long blocks first: work is concentrated in few tiles, and a frame ends
+    // with the long blocks sharing their SIMDs
+    const uint32_t len = end - lo;
+    if (len >= 256u)
+        __builtin_amdgcn_s_setprio(3);
+    else if (len >= 128u)
+        __builtin_amdgcn_s_setprio(2);
+    else if (len >= 64u)
+        __builtin_amdgcn_s_setprio(1);
+    const float wf = (float)img_w, hf = (float)img_h;
+    // the refine weight |(W vx, H vy)| / A with (vx, vy) = v_sigma ln2 (gx, gy)
+    const float refine_scale = kLn2 * __builtin_amdgcn_rcpf(bh_maxf(final_a, 1.0e-5f));
+    const size_t rbase = REPLAY ? 0 : record_base<BPT>(blk, lo, hi) - lo;
+    const float bx0 = (float)((tile % tile_bw) * 16u + (blk & 1u) * 8u) + 0.5f;
+    const float by0 = (float)((tile / tile_bw) * (uint32_t)TH + (blk >> 1) * 8u) + 0.5f;
+    // pixels outside the image and, with REPLAY, those that have saturated
+    uint64_t dead = __builtin_amdgcn_ballot_w64(!inside);
+
+    // a step's sums end in lane 16 r + 4 a + k (value 4 a + r with the bits of
+    // r swapped, of the lane's own candidate); the lanes past the values add
+    // into slot NB's row
+    const uint32_t sum_value = (lane & 12u) + ((lane >> 4) & 1u) * 2u + (lane >> 5);
+    const bool sums = sum_value < (uint32_t)K;
+    const uint32_t sum_mul = sums ? GS / 4u : 0u;  // of a record's byte offset
+    char* const sum_to = sums ? reinterpret_cast<char*>(&s_sum[sub][sum_value]) : reinterpret_cast<char*>(&s_dump[lane]);
+    // what multiplies a total when it leaves the workgroup (lane 16 r + j,
+    // value j): its own total times c00 (v_sigma dx), c11 (v_sigma dy), 0.5
+    // (dx dx and dy dy), the colour gate (a colour) or 1, plus the other mean
+    // row's total times c01
+    const uint32_t fk = t & 15u;
+    const float f00 = fk == 0u ? kTwoLn2 : 0.0f, f11 = fk == 1u ? kTwoLn2 : 0.0f;
+    const float f01 = fk < 2u ? kLn2 : 0.0f;
+    const uint32_t fgate = fk >= 5u && fk <= 7u ? 1u << (fk - 5u) : 0u;
+    const float fconst = fk < 2u || fgate ? 0.0f : ((fk == 2u || fk == 4u) ? 0.5f : 1.0f);
+    const uint32_t fdst = fk < 9u ? fk : (fk == 9u && REFINE ? 9u : 10u);
+    if (t == 0u) {
+        s_geo[NB] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        s_op[NB] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        s_aux[NB] = make_uint4(0u, 0u, 0u, 0u);
+        s_mask[NB] = 0ull;
+    }
+
+    // The first two waves stage a batch.  Its rows are read while the one
+    // before it is evaluated, its masks and ids one batch earlier still.
+    const uint32_t last = end - 1u;
+    const bool stages = sub < NB / 64u;
+    uint64_t mask = 0ull;  // of the batch about to be staged
+    uint2 mask_n = make_uint2(0u, 0u);
+    uint32_t cid_n = 0u, grow = 0u;
+    float2 r0, r1, r2, r3, r4;
+    auto load_masks = [&](uint32_t b) {
+        const uint32_t i = min(b + t, last);
+        if (!REPLAY) mask_n = rec.masks[rbase + i];
+        cid_n = cgids[i];
+    };
+    auto load_rows = [&](uint32_t b) {  // of the batch at b, whose masks have arrived
+        mask = b + t <= last ? (REPLAY ? 1ull : ((uint64_t)mask_n.y << 32) | mask_n.x) : 0ull;
+        if (mask) {
+            const uint32_t c = min(cid_n, num_visible - 1u);
+            const float2* prow = reinterpret_cast<const float2*>(projected + (size_t)c * 10);
+            r0 = prow[0], r1 = prow[1], r2 = prow[2], r3 = prow[3], r4 = prow[4];
+            grow = row_of ? row_of[c] : c;
+        }
+    };
+    if (stages) {
+        load_masks(lo);
+        load_rows(lo);
+        load_masks(lo + NB);
+    }
+    for (uint32_t b = lo; b < end; b += NB) {
+        if (stages) {
+            float cut = 0.0f;
+            if (REPLAY && mask) {
+                cut = sigma_cutoff<SMOOTH>(r2.y);
+                const uint32_t m = touches_sub_blocks(r0.x, r0.y, S2{r1.x, r1.y, r2.x}, cut, bx0, by0);
+                mask = (uint64_t)(m & 1u) | (uint64_t)(m & 2u) << 15 | (uint64_t)(m & 4u) << 30 | (uint64_t)(m & 8u) << 45;
+            }
+            s_mask[t] = mask;
+            if (mask) {
+                float ka, kb, kc;
+                bh_conic_log2(r1.x, r1.y, r2.x, &ka, &kb, &kc);
+                s_geo[t] = make_float4(r0.x, r0.y, ka, kb);
+                s_op[t] = make_float4(kc, r2.y, bh_maxf(r3.x, 0.0f), bh_maxf(r3.y, 0.0f));
+                // the cutoff's margin of 1e-3 covers the rounding of the scaled power
+                s_aux[t] = make_uint4(__float_as_uint(bh_maxf(r4.x, 0.0f)), __float_as_uint(kLog2e * cut),
+                                      (r3.x >= 0.0f ? 1u : 0u) | (r3.y >= 0.0f ? 2u : 0u) | (r4.x >= 0.0f ? 4u : 0u),
+                                      grow);
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 5u; i++) {
+                const uint64_t m = __builtin_amdgcn_ballot_w64(
+                    i < 4u ? ((mask >> (16u * (i & 3u))) & 0xFFFFull) != 0ull : mask != 0ull);
+                if (lane == i) s_touch[i][sub] = m;
+            }
+            if (b + NB < end) {
+                load_rows(b + NB);
+                load_masks(b + 2u * NB);
+            }
+        }
+        __syncthreads();
+        auto wave_mask = [&](uint32_t i, uint32_t w) {
+            const unsigned long long v = s_touch[i][w];
+            return ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+                   (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+        };
+        // the block's candidates, and this sub-block's (byte offsets of the
+        // 16-byte records)
+        uint32_t n_any = 0u, n = 0u;
+#pragma unroll
+        for (uint32_t w = 0; w < NB / 64u; w++) {
+            const uint64_t ma = wave_mask(4u, w), m = wave_mask(sub, w);
+            if (w == sub && ((ma >> lane) & 1ull)) s_any[n_any + lanes_below(ma)] = (uint16_t)t;
+            n_any += (uint32_t)__popcll(ma);
+            if ((m >> lane) & 1ull) s_list[sub][n + lanes_below(m)] = (uint16_t)((w * 64u + lane) * 16u);
+            n += (uint32_t)__popcll(m);
+        }
+        if (lane < 16u) s_list[sub][n + lane] = (uint16_t)(NB * 16u);
+        wave_lds_fence();
+        const uint32_t steps = (n + 3u) >> 2;
+        const uint16_t* list = &s_list[sub][slot];
+        struct Set {
+            float4 geo, op;
+            float cb;
+            uint32_t mask;  // (REPLAY: the cutoff's bits)
+        };
+        auto fetch = [&](uint32_t off, Set& s) {
+            s.geo = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_geo) + off);
+            s.op = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_op) + off);
+            const uint32_t* aux = reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(s_aux) + off);
+            s.cb = __uint_as_float(aux[0]);
+            s.mask = REPLAY ? aux[1]
+                            : *reinterpret_cast<const uint16_t*>(reinterpret_cast<const char*>(s_mask) + (off >> 1) +
+                                                                 sub * 2u);
+        };
+        // four candidates front to back
+        auto eval_four = [&](const Set& s, uint32_t off) {
+            const float ka = s.geo.z, kb = s.geo.w, kc = s.op.x, opac = s.op.y;
+            const float cr = s.op.z, cg = s.op.w, cb = s.cb;
+            // d = mean - pixel centre; the forward's power and Gaussian, bit
+            // for bit
+            const float dx = s.geo.x - pcx, dy = s.geo.y - pcy;
+            const float power = bh_power_log2(ka, kb, kc, dx, dy);
+            const float gauss = bh_exp2_neg(-power);
+            const float og = opac * gauss;
+            const float alpha = bh_minf(0.999f, og);
+            float w = 1.0f, ae = alpha;
+            if (SMOOTH) {
+                w = cutoff_weight(alpha);
+                ae = alpha * w;
+            }
+            // the record's bit, or whether the pair passes the cutoff
+            bool contrib;
+            if constexpr (REPLAY)
+                contrib = __builtin_amdgcn_inverse_ballot_w64(
+                    __builtin_amdgcn_ballot_w64(power >= 0.0f) &
+                    __builtin_amdgcn_ballot_w64(!(power > __uint_as_float(s.mask))) &
+                    (SMOOTH ? __builtin_amdgcn_ballot_w64(w > 0.0f) : __builtin_amdgcn_ballot_w64(alpha >= kCutMid)));
+            else
+                contrib = ((s.mask >> p) & 1u) != 0u;
+            ae = contrib ? ae : 0.0f;
+            float om = 1.0f - ae;
+            // the forward's transmittances, factor by factor
+            float n0 = sw * quad_f32<0>(om), n1 = n0 * quad_f32<1>(om);
+            float n2 = n1 * quad_f32<2>(om), n3 = n2 * quad_f32<3>(om);
+            float own_t = quad_pick(sw, n0, n1, n2);
+            if constexpr (REPLAY) {
+                if ((__builtin_amdgcn_ballot_w64(n3 > 1.0e-4f) | dead) != ~0ull) {
+                    // some pixel saturates in this step: it blends neither that
+                    // candidate nor a later one, and its transmittance is 0
+                    // from there on
+                    auto next = [](float tt, float omk) {
+                        const float x = tt * omk;
+                        return x > 1.0e-4f ? x : 0.0f;
+                    };
+                    n0 = next(sw, quad_f32<0>(om));
+                    n1 = next(n0, quad_f32<1>(om));
+                    n2 = next(n1, quad_f32<2>(om));
+                    n3 = next(n2, quad_f32<3>(om));
+                    own_t = quad_pick(sw, n0, n1, n2);
+                    contrib = contrib && quad_pick(n0, n1, n2, n3) > 0.0f;
+                    ae = contrib ? ae : 0.0f;
+                    om = 1.0f - ae;
+                    dead = __builtin_amdgcn_ballot_w64(n3 == 0.0f);
+                } else {
+                    contrib = contrib && own_t > 0.0f;
+                }
+            }
+            sw = n3;
+            const float vis = ae * own_t;
+            // position, conic, opacity and refine lanes: contributing and
+            // unclamped pairs (o G <= 0.999); the selects sit on v_sigma and on
+            // the opacity lane, so other lanes' values never reach a sum
+            const bool gate = contrib && og <= 0.999f;
+            float g[K];
+            {
+#pragma clang fp contract(fast)
+                // gradient-only arithmetic: products and sums fuse into FMAs
+                const float ra = __builtin_amdgcn_rcpf(om);
+                const float cv = cr * vox + cg * voy + cb * voz;
+                // the reference's state update (rasterize_backwards.rs:356-358,
+                // 432-435) as D -= vis (c . v_out)
+                const float q = vis * cv;
+                const float d1 = dsum - quad_f32<0>(q), d2 = d1 - quad_f32<1>(q), d3 = d2 - quad_f32<2>(q);
+                const float own_d = quad_pick(dsum, d1, d2, d3);
+                dsum = d3 - quad_f32<3>(q);
+                // ((T c - S) . v_out + v_ow) / (1 - alpha)
+                const float v_ae = (own_t * cv - own_d + vow) * ra;
+                const float v_alpha = SMOOTH ? v_ae * (w + alpha * cutoff_weight_deriv(alpha)) : v_ae;
+                const float v_sigma = gate ? -alpha * v_alpha : 0.0f;
+                const float tx = v_sigma * dx, ty = v_sigma * dy;
+                g[0] = tx;
+                g[1] = ty;
+                g[2] = tx * dx;
+                g[3] = tx * dy;
+                g[4] = ty * dy;
+                g[5] = vis * vox;
+                g[6] = vis * voy;
+                g[7] = vis * voz;
+                g[8] = gate ? v_alpha * gauss : 0.0f;
+                if constexpr (REFINE) {
+                    // (vx, vy) = v_sigma C d = v_sigma ln2 (gx, gy) with
+                    // gx = 2 a dx + b dy = q + a dx (q = a dx + b dy of the
+                    // power) and gy = b dx + 2 c dy
+                    const float qq = bh_fmaf(ka, dx, kb * dy);
+                    const float cdy = kc * dy;
+                    const float gx = bh_fmaf(ka, dx, qq), gy = bh_fmaf(kb, dx, cdy + cdy);
+                    const float ax = wf * gx, ay = hf * gy;
+                    g[9] = (__builtin_fabsf(v_sigma) * refine_scale) * __builtin_amdgcn_sqrtf(ax * ax + ay * ay);
+                }
+                if constexpr (DEPTH) g[K - 1] = vis * vod;
+            }
+            // values 4 j .. 4 j + 3 folded into one register over the lanes'
+            // upper bits (rows r hold values 4 j + 0, 2, 1, 3), summed over the
+            // row's four pixels, and register j kept in the lanes a = j
+            float q[3];
+#pragma unroll
+            for (int j = 0; j < 3; ++j) {
+                const float v0 = g[4 * j], v1 = g[4 * j + 1];
+                const float v2 = 4 * j + 2 < K ? g[4 * j + 2 < K ? 4 * j + 2 : 0] : 0.0f;
+                const float v3 = 4 * j + 3 < K ? g[4 * j + 3 < K ? 4 * j + 3 : 0] : 0.0f;
+                const float hi = 4 * j + 2 < K ? psum32(v2, v3) : 0.0f;
+                q[j] = psum16(psum32(v0, v1), hi);
+                q[j] = dpp_add<0x124>(q[j]);  // row_ror:4
+                q[j] = dpp_add<0x128>(q[j]);  // row_ror:8
+            }
+            float tot = q[0];
+            tot = __builtin_amdgcn_inverse_ballot_w64(0x00F000F000F000F0ull) ? q[1] : tot;
+            tot = __builtin_amdgcn_inverse_ballot_w64(0x0F000F000F000F00ull) ? q[2] : tot;
+            *reinterpret_cast<float*>(sum_to + __umul24(off, sum_mul)) = tot;
+        };
+        uint32_t done = 0u;  // candidates of the list evaluated
+        if (steps && (!REPLAY || dead != ~0ull)) {
+            // the next step's parameters are read while one is evaluated, its
+            // indices a step earlier, two register sets in turn
+            Set sa, sb;
+            uint32_t oa = list[0], ob = list[4];
+            fetch(oa, sa);
+            for (uint32_t i = 0;; i += 2u) {
+                const uint32_t oc = list[4u * i + 8u];
+                fetch(ob, sb);
+                eval_four(sa, oa);
+                done = 4u * i + 4u;
+                if (i + 1u >= steps || (REPLAY && dead == ~0ull)) break;
+                const uint32_t od = list[4u * i + 12u];
+                fetch(oc, sa);
+                eval_four(sb, ob);
+                done = 4u * i + 8u;
+                if (i + 2u >= steps || (REPLAY && dead == ~0ull)) break;
+                oa = oc;
+                ob = od;
+            }
+        }
+        if (REPLAY) {
+            // the sums of the candidates behind the last live pixel are zero
+            for (uint32_t i = done + lane; i < n; i += 64u) {
+                float* z = &s_sum[sub][s_list[sub][i] / 16u * GS];
+#pragma unroll
+                for (int j = 0; j < K; ++j) z[j] = 0.0f;
+            }
+            if (lane == 0u) s_alive[sub] = dead != ~0ull ? 1u : 0u;
+        }
+        __syncthreads();
+        // the block's sums, sixteen threads a candidate (the trip count is
+        // uniform: the mean rows exchange totals over the lanes)
+        for (uint32_t i = t >> 4; i - (t >> 4) < n_any; i += 16u) {
+            const bool live = i < n_any && fk < (uint32_t)K;
+            const uint32_t c = s_any[live ? i : 0u];
+            const uint64_t m = s_mask[c];
+            float own = 0.0f;
+#pragma unroll
+            for (uint32_t q = 0; q < 4u; q++)
+                if (live && ((m >> (16u * q)) & 0xFFFFull)) own += s_sum[q][c * GS + fk];
+            const float other = __uint_as_float(quad_xor1_u32(__float_as_uint(own)));
+            if (live) {
+                const uint4 aux = s_aux[c];
+                const float fself = f00 * s_geo[c].z + (f11 * s_op[c].x + (fconst + ((aux.z & fgate) ? 1.0f : 0.0f)));
+                const float v = f01 != 0.0f ? fself * own + (f01 * s_geo[c].w) * other : fself * own;
+                if (v != 0.0f) unsafeAtomicAdd(v_rows + (size_t)aux.w * kNG + fdst, v);
+            }
+        }
+        const bool over = REPLAY && (s_alive[0] | s_alive[1] | s_alive[2] | s_alive[3]) == 0u;
+        __syncthreads();
+        if (over) break;
+    }
+}
+
+
+void launch_rasterize_backward(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile_bw, uint32_t tile_bh,
+                               const float* bg, uint32_t num_visible, const float* out_img, const float* projected, const uint32_t* cgids,
+                               const uint32_t* offsets, const float* v_output, uint32_t flags,
+                               const uint32_t* row_of, const uint32_t* order, float* v_combined) {
+    const uint32_t num_tiles = tile_bw * tile_bh;
+    if (num_tiles == 0 || num_visible == 0) return;
+    const bool smooth = (flags & BH_FLAG_SMOOTH_CUTOFF) != 0;
+    const bool refine = (flags & BH_FLAG_REFINE_WEIGHT) != 0;
+    const bool depth = (flags & BH_FLAG_RENDER_DEPTH) != 0;
+    const bool fine = (flags & BH_FLAG_TILE_16X8) != 0;
+    const uint32_t groups = div_up(num_tiles, 8) * (fine ? 16u : 32u);
+    KernelTimer t(ctx, "rasterize_backward");
+#define BH_RB_T(S, R, D, T)                                                                                        \
+    launch(ctx, rasterize_backward_quad_kernel<true, S, R, D, T>, dim3(groups), dim3(256), 0u, img_w, img_h, tile_bw,   \
+           num_tiles, bg[0], bg[1], bg[2], num_visible, out_img, projected, cgids, offsets, SplatRecord{}, v_output, \
+           row_of, order, v_combined, FillRanges{}, 0u, 0u)
+#define BH_RB(S, R, D) \
+    do {               \
+        if (fine)      \
+            BH_RB_T(S, R, D, 8); \
+        else           \
+            BH_RB_T(S, R, D, 16); \
+    } while (0)
+    if (smooth) {
+        if (refine) {
+            if (depth) BH_RB(true, true, true); else BH_RB(true, true, false);
+        } else {
+            if (depth) BH_RB(true, false, true); else BH_RB(true, false, false);
+        }
+    } else {
+        if (refine) {
+            if (depth) BH_RB(false, true, true); else BH_RB(false, true, false);
+        } else {
+            if (depth) BH_RB(false, false, true); else BH_RB(false, false, false);
+        }
+    }
+#undef BH_RB_T
+#undef BH_RB
+}
 
 template <bool S, bool R, bool D, int T>
 static void launch_recorded_t(bh_ctx* ctx, uint32_t groups, uint32_t img_w, uint32_t img_h, uint32_t tile_bw,
@@ -717,17 +935,19 @@ static void launch_recorded_t(bh_ctx* ctx, uint32_t groups, uint32_t img_w, uint
                               const SplatRecord& rec, const float* v_output, const uint32_t* row_of,
                               const uint32_t* order, float* v_rows, const FillRanges& fill, uint32_t fill_slots) {
     const uint32_t all_slots = groups / 8u + fill_slots;
-    launch(ctx, rasterize_backward_recorded_kernel<S, R, D, T>, dim3(all_slots * 8u), dim3(64), 0u, img_w, img_h,
-           tile_bw, num_tiles, bg[0], bg[1], bg[2], num_visible, out_img, projected, cgids, off_pre, rec, v_output,
-           row_of, order, v_rows, fill, fill_slots, all_slots);
+    if (backward_in_quads(num_tiles, T == 8))
+        launch(ctx, rasterize_backward_quad_kernel<false, S, R, D, T>, dim3(all_slots * 8u), dim3(256), 0u, img_w, img_h,
+               tile_bw, num_tiles, bg[0], bg[1], bg[2], num_visible, out_img, projected, cgids, off_pre, rec, v_output,
+               row_of, order, v_rows, fill, fill_slots, all_slots);
+    else
+        launch(ctx, rasterize_backward_recorded_kernel<S, R, D, T>, dim3(all_slots * 8u), dim3(64), 0u, img_w, img_h,
+               tile_bw, num_tiles, bg[0], bg[1], bg[2], num_visible, out_img, projected, cgids, off_pre, rec, v_output,
+               row_of, order, v_rows, fill, fill_slots, all_slots);
 }
 
 // 16-byte stores per lane of a workgroup that zeroes the fill ranges inside the
 // rasterize backward (about 64 KiB a workgroup)
-#ifndef BH_FUSED_FILL_ITERS
-#define BH_FUSED_FILL_ITERS 64
-#endif
-constexpr uint64_t kFusedFillIters = BH_FUSED_FILL_ITERS;
+constexpr uint64_t kFusedFillIters = 64;
 
 bool launch_rasterize_backward_recorded(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile_bw,
                                         uint32_t tile_bh, const float* bg, uint32_t num_visible, const float* out_img,

@@ -325,6 +325,21 @@ void launch_zero_and_tile_order(bh_ctx* ctx, uint32_t* p, uint64_t words, const 
 // pairs for the fused backward (bh_splat_record.h), and with rec.order.list
 // the backward's dispatch order.  With BWD_INFO, workgroups after the blend's
 // zero fill[0, fill_words) (16-byte aligned) in its tail.
+// Whether a frame's blend, or its fused rasterize backward, runs a workgroup of
+// four waves per 8x8 block (a 4x4 sub-block each, four candidates per step)
+// instead of one wave.  With few blocks one wave each leaves the chip idle, and
+// the frame waits for its longest blocks; with many the chip is full, and the
+// four waves' 1.4-1.5 times the instructions cost.  Where the lines lie: the
+// blend at 4,800 blocks (640x480) takes 66 -> 37 us, 83 -> 46 us (clusters)
+// and 59 -> 67 us (every tile loaded alike), at 7,600 57 -> 42, 78 -> 48 and
+// 104 -> 127 us; the backward at 7,600 93 -> 64, 126 -> 75 and 225 -> 235 us,
+// at 12,288 85 -> 82, 107 -> 96 and 279 -> 335 us.
+inline bool blend_in_quads(uint32_t num_tiles, bool fine) {
+    return num_tiles * (fine ? 2u : 4u) <= 6144u;
+}
+inline bool backward_in_quads(uint32_t num_tiles, bool fine) {
+    return num_tiles * (fine ? 2u : 4u) <= 8192u;
+}
 void launch_rasterize(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile_bw, uint32_t tile_bh,
                       const float* bg, uint32_t num_visible, const float* projected, const uint32_t* cgids,
                       const uint32_t* gfc, const uint32_t* off_pre, const uint32_t* order, uint32_t flags,

@@ -12,15 +12,15 @@
 //
 // Layout, per 8x8 block of a tile whose candidate list is [lo, hi) (len =
 // hi - lo, BPT blocks per tile):
-//   masks[BPT lo + blk len + (k - lo)]  bit p: candidate k contributed to
-//                                       pixel p of the block (p = lane =
-//                                       x + 8 y within the block)
+//   masks[BPT lo + blk len + (k - lo)]  bit 16 s + p: candidate k contributed
+//                                       to pixel p = x + 4 y of the block's 4x4
+//                                       sub-block s = sx + 2 sy
 //   block_end[tile BPT + blk]           one past the last candidate any
 //                                       pixel of the block consumed (lo when
 //                                       none did)
 // Candidate runs are in tile order, so the tiles' regions [BPT lo, BPT hi)
 // partition [0, BPT M) (M candidates).  The forward writes the masks of every
-// batch of 64 candidates it walks; the backward reads candidates below
+// batch of candidates it walks; the backward reads candidates below
 // block_end only, all of which lie in walked batches.
 #pragma once
 

@@ -2,21 +2,23 @@
 //
 //   tile_offsets  [start, end) of each tile's run in the tile-sorted list
 //                 (crates/brush-render/src/get_tile_offset.rs:10-62)
-//   rasterize     one single-wave workgroup per 8x8 pixel block of a 16x16
-//                 tile, one pixel per lane; each wave stages the tile's splats
-//                 in LDS in batches of 64, keeps those that may touch its block
-//                 (ballot of a conservative rectangle test) and stops when its
-//                 64 pixels have saturated
-//                 (crates/brush-render/src/kernels/rasterize.rs:24-200).
+//   rasterize     the blend by 8x8 pixel blocks of a 16x16 tile
+//                 (crates/brush-render/src/kernels/rasterize.rs:24-200): one
+//                 wave per block, one pixel per lane, a candidate at a time
+//                 (rasterize_kernel), or in small frames four waves per block,
+//                 a 4x4 sub-block and four candidates at a time each
+//                 (rasterize_quad_kernel).  The tile's splats are staged in
+//                 LDS in batches, those that may touch the block kept (ballot
+//                 of a conservative rectangle test), until its 64 pixels have
+//                 saturated.
 //
 // With BWD_INFO the kernel also marks contributing splats visible — once per
-// (splat, block) through a ballot instead of once per pixel — and shrinks each
+// (splat, block) instead of once per pixel — and shrinks each
 // tile's end to one past the last splat any pixel consumed (an atomic max over
 // the tile's four blocks).  It also records which pairs contributed, for the
 // fused backward (bh_splat_record.h): per block and candidate, the 64-bit mask
-// of the block's pixels that blended it (the ballot of the blend decision,
-// moved into the candidate's lane), and per block the end of the candidates its
-// pixels consumed.
+// of the block's pixels that blended it, and per block the end of the
+// candidates its pixels consumed.
 #include <hip/hip_runtime.h>
 
 #include "bh_internal.h"
@@ -76,6 +78,20 @@ void launch_tile_offsets(bh_ctx* ctx, const uint32_t* tile_ids, uint32_t m, uint
 extern "C" __device__ int bh_llvm_writelane(int value, int lane, int old) __asm("llvm.amdgcn.writelane.i32");
 __device__ __forceinline__ uint32_t write_lane(uint32_t old, uint32_t value, uint32_t lane) {
     return (uint32_t)bh_llvm_writelane((int)value, (int)lane, (int)old);
+}
+
+// acc += v_k c[k] for the quad's lanes k = 0..3 in turn, v_k being lane k's v
+// (fused, in that order).  Written out because the compiler broadcasts v into
+// registers first; the leading wait states are those a DPP read of a register
+// that the instruction before it may have written needs.
+__device__ __forceinline__ void quad_fma4(float& acc, float v, const float (&c)[4]) {
+    __asm__("s_nop 1\n\t"
+            "v_fmac_f32_dpp %0, %1, %2 quad_perm:[0,0,0,0] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, %1, %3 quad_perm:[1,1,1,1] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, %1, %4 quad_perm:[2,2,2,2] row_mask:0xf bank_mask:0xf\n\t"
+            "v_fmac_f32_dpp %0, %1, %5 quad_perm:[3,3,3,3] row_mask:0xf bank_mask:0xf"
+            : "+v"(acc)
+            : "v"(v), "v"(c[0]), "v"(c[1]), "v"(c[2]), "v"(c[3]));
 }
 
 // One workgroup (a single wave) per 8x8 pixel block of a 16 x TH tile; the
@@ -228,6 +244,7 @@ void launch_zero_and_tile_order(bh_ctx* ctx, uint32_t* p, uint64_t words, const 
            order);
 }
 
+// 16-byte stores per lane of a trailing zero-fill workgroup
 constexpr uint32_t kFillQuadsPerLane = 16;
 
 template <bool BWD_INFO, bool SMOOTH, bool DEPTH, int TH>
@@ -268,7 +285,8 @@ __global__ __launch_bounds__(64) void rasterize_kernel(uint32_t img_w, uint32_t 
     const uint32_t lane = threadIdx.x;
     const uint32_t ox = (tile % tile_bw) * 16u + (blk & 1u) * 8u;
     const uint32_t oy = (tile / tile_bw) * (uint32_t)TH + (blk >> 1) * 8u;
-    const uint32_t px = ox + (lane & 7u), py = oy + (lane >> 3);
+    // lane 16 s + p: pixel p of 4x4 sub-block s (the record's bit order)
+    const uint32_t px = ox + ((lane >> 4) & 1u) * 4u + (lane & 3u), py = oy + (lane >> 5) * 4u + ((lane >> 2) & 3u);
     const bool inside = px < img_w && py < img_h;
     const uint32_t lo = off_pre[2 * tile], hi = off_pre[2 * tile + 1];
     // Long blocks first: the wave priority rises with the tile's candidate
@@ -333,8 +351,7 @@ __global__ __launch_bounds__(64) void rasterize_kernel(uint32_t img_w, uint32_t 
         // the cutoff's margin of 1e-3 covers the rounding of the scaled power
         s_c11a[lane] = make_float4(kc, cc.y, kLog2e * cut, 0.0f);
         s_rgbd[lane] = make_float4(staged_colour(d.x), staged_colour(d.y), staged_colour(e.x), e.y);
-        const bool touch = lane < cnt && may_touch_rect(a.x, a.y, S2{b.x, b.y, cc.x}, cut, bx0, by0, bx0 + 7.0f,
-                                                        by0 + 7.0f);
+        const bool touch = lane < cnt && touches_block(a.x, a.y, S2{b.x, b.y, cc.x}, cut, bx0, by0);
         // splats of the batch that may touch this block, in order
         uint64_t todo = __builtin_amdgcn_ballot_w64(touch);
         mask_lo = 0u;
@@ -475,6 +492,324 @@ __global__ __launch_bounds__(64) void rasterize_kernel(uint32_t img_w, uint32_t 
     }
 }
 
+// Candidates staged per batch, one per thread of the workgroup.
+constexpr uint32_t kBlendBatch = 256;
+
+// The blend.  A workgroup owns one 8x8 pixel block of a 16 x TH tile; each of
+// its four waves one 4x4 sub-block, lane 4 p + k holding pixel p (x + 4 y in
+// the sub-block) and the k-th of the four candidates the wave takes per step.
+// A pair's alpha is evaluated once, by its own lane; the front-to-back chain
+// over the four candidates (transmittance, saturation, the colour sums, lane
+// k's being channel k) runs in every lane of a pixel's quad over DPP
+// broadcasts, in the order and with the roundings of a per-pixel walk.
+//
+// What bounds it: with few blocks the chip is not full, and a block's time is
+// the issue of its own instructions (a wave retires one every five to nine
+// cycles, whatever its kind).  One wave per 8x8 block, a candidate per step,
+// takes ~45 VALU a candidate; a step here takes ~58 for four, of a quarter of
+// the pixels, and a 4x4 sub-block skips the candidates that touch only its
+// neighbours (100k splats at 256x256: 116 blended candidates per 4x4 against
+// 183 per 8x8 block).  The workgroup stages 256 candidates at a time, so the
+// staging (a logarithm, the touch tests) is shared by four waves.  One wave
+// per block -> four: 96x64, 4k splats 102 -> 32 us, 256x256, 100k 103 -> 43 us,
+// 640x360, 250k 65 -> 36 us (event times).  A full chip issues 1.5 times the
+// instructions (1920x1080: 70M VALU against 42M, 86 -> 138 us), so
+// blend_in_quads draws the line.
+template <bool BWD_INFO, bool SMOOTH, bool DEPTH, int TH>
+__global__ __launch_bounds__(256, 5) void rasterize_quad_kernel(uint32_t img_w, uint32_t img_h, uint32_t tile_bw,
+                                                         uint32_t num_tiles, float bg_r, float bg_g, float bg_b,
+                                                         uint32_t num_visible, const float* __restrict__ projected,
+                                                         const uint32_t* __restrict__ cgids,
+                                                         const uint32_t* __restrict__ gfc,
+                                                         const uint32_t* __restrict__ off_pre,
+                                                         const uint32_t* __restrict__ order,
+                                                         void* __restrict__ out_img, float* __restrict__ visible,
+                                                         uint32_t* __restrict__ off_post, SplatRecord rec,
+                                                         uint32_t* __restrict__ fill, uint64_t fill_words,
+                                                         uint32_t blend_groups) {
+    constexpr uint32_t NB = kBlendBatch;
+    // slot NB is a splat of opacity 0 that pads a step of fewer than four
+    __shared__ float4 s_geo[NB + 1];  // x, y and the scaled conic a, b (bh_conic_log2)
+    __shared__ float4 s_op[NB + 1];   // scaled conic c, opacity, cutoff on the power in base 2
+    __shared__ float4 s_col[NB + 1];  // r, g, b (staged_colour), depth
+    __shared__ unsigned long long s_touch[4][4];  // [sub-block][staging wave]
+    __shared__ uint16_t s_list[4][NB + 16];       // each sub-block's candidates, in order
+    __shared__ unsigned long long s_bal[BWD_INFO ? 4 : 1][NB / 4];  // contributing pairs of each step
+    __shared__ unsigned long long s_mask[BWD_INFO ? NB : 1];        // ... of each candidate (bh_splat_record.h)
+    __shared__ uint32_t s_alive[4], s_last[4];
+
+    const uint32_t t = threadIdx.x;
+    if (BWD_INFO && blockIdx.x >= blend_groups) {
+        // the backward's gradient rows: 64 KB per trailing workgroup, which
+        // the dispatcher starts as the blend's blocks drain
+        const uint64_t q0 = (uint64_t)(blockIdx.x - blend_groups) * (256u * kFillQuadsPerLane);
+        uint4* q = reinterpret_cast<uint4*>(fill);
+        const uint64_t quads = fill_words / 4u;
+#pragma unroll
+        for (uint32_t k = 0; k < kFillQuadsPerLane; k++) {
+            const uint64_t i = q0 + k * 256u + t;
+            if (i < quads) q[i] = make_uint4(0u, 0u, 0u, 0u);
+        }
+        if (q0 == 0u && t < fill_words % 4u) fill[quads * 4u + t] = 0u;
+        return;
+    }
+    uint32_t tile, blk;
+    raster_block_of_workgroup<TH>(blockIdx.x, tile, blk);
+    if (tile >= num_tiles) return;
+    if (order) tile = order[tile];
+    const uint32_t lane = t & 63u, sub = (uint32_t)__builtin_amdgcn_readfirstlane((int)(t >> 6));
+    const uint32_t slot = lane & 3u, p = lane >> 2;
+    const uint32_t ox = (tile % tile_bw) * 16u + (blk & 1u) * 8u;
+    const uint32_t oy = (tile / tile_bw) * (uint32_t)TH + (blk >> 1) * 8u;
+    const uint32_t px = ox + (sub & 1u) * 4u + (p & 3u), py = oy + (sub >> 1) * 4u + (p >> 2);
+    const bool inside = px < img_w && py < img_h;
+    const uint32_t lo = off_pre[2 * tile], hi = ox < img_w && oy < img_h ? off_pre[2 * tile + 1] : lo;
+    // Long blocks first: the wave priority rises with the tile's candidate
+    // count (work is concentrated in few tiles; see the backward kernel).
+    const uint32_t len = hi - lo;
+    if (len >= 6144u)
+        __builtin_amdgcn_s_setprio(3);
+    else if (len >= 3072u)
+        __builtin_amdgcn_s_setprio(2);
+    else if (len >= 1024u)
+        __builtin_amdgcn_s_setprio(1);
+    const float pcx = (float)px + 0.5f, pcy = (float)py + 0.5f;
+    const float bx0 = (float)ox + 0.5f, by0 = (float)oy + 0.5f;
+    // the pixel's transmittance while it lives (0 from its saturation on), the
+    // one it kept at saturation, and this lane's channel sum
+    float t_live = inside ? 1.0f : 0.0f, t_kept = 1.0f, acc = 0.0f;
+    uint64_t dead = __builtin_amdgcn_ballot_w64(!inside);
+    uint32_t last = lo;
+    constexpr uint32_t BPT = 2u * (uint32_t)TH / 8u;
+    const size_t rbase = BWD_INFO ? record_base<BPT>(blk, lo, hi) : 0;
+    if (t == 0u) {
+        s_geo[NB] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        s_op[NB] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        s_col[NB] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    }
+
+    // A batch's rows are read while the one before it is blended, its ids one
+    // batch earlier still (unconditional reads, at indices clamped into the run).
+    const uint32_t lastc = hi - 1u;
+    float2 ra, rb, rc, rd, re;
+    uint32_t gid = 0u, gid_n = 0u, cid_n = 0u;
+    auto load_rows = [&](uint32_t c) {
+        c = min(c, num_visible - 1u);
+        const float2* row = reinterpret_cast<const float2*>(projected + (size_t)c * 10);
+        ra = row[0], rb = row[1], rc = row[2], rd = row[3], re = row[4];
+        if (BWD_INFO) gid_n = gfc[c];
+    };
+    if (hi > lo) {
+        load_rows(cgids[min(lo + t, lastc)]);
+        cid_n = cgids[min(lo + NB + t, lastc)];
+    }
+    for (uint32_t batch = lo; batch < hi; batch += NB) {
+        // a block still blending after 256 candidates is one of the long ones
+        // whatever its candidate count said: top priority from here on
+        if (batch == lo + NB) __builtin_amdgcn_s_setprio(3);
+        const float cut = sigma_cutoff<SMOOTH>(rc.y);
+        float ka, kb, kc;
+        bh_conic_log2(rb.x, rb.y, rc.x, &ka, &kb, &kc);
+        s_geo[t] = make_float4(ra.x, ra.y, ka, kb);
+        // the cutoff's margin of 1e-3 covers the rounding of the scaled power
+        s_op[t] = make_float4(kc, rc.y, kLog2e * cut, 0.0f);
+        s_col[t] = make_float4(staged_colour(rd.x), staged_colour(rd.y), staged_colour(re.x), re.y);
+        if (BWD_INFO) s_mask[t] = 0ull;
+        const uint32_t touch =
+            batch + t < hi ? touches_sub_blocks(ra.x, ra.y, S2{rb.x, rb.y, rc.x}, cut, bx0, by0) : 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4u; i++) {
+            const uint64_t m = __builtin_amdgcn_ballot_w64(((touch >> i) & 1u) != 0u);
+            if (lane == i) s_touch[i][sub] = m;
+        }
+        gid = gid_n;
+        if (batch + NB < hi) {
+            load_rows(cid_n);
+            cid_n = cgids[min(batch + 2u * NB + t, lastc)];
+        }
+        __syncthreads();
+        if (dead != ~0ull) {
+            // this sub-block's candidates of the batch, in order
+            uint32_t n = 0u;
+#pragma unroll
+            for (uint32_t w = 0; w < 4u; w++) {
+                const unsigned long long v = s_touch[sub][w];
+                const uint64_t m = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(v >> 32)) << 32) |
+                                   (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)v);
+                if ((m >> lane) & 1ull) s_list[sub][n + lanes_below(m)] = (uint16_t)((w * 64u + lane) * 16u);
+                n += (uint32_t)__popcll(m);
+            }
+            if (lane < 16u) s_list[sub][n + lane] = (uint16_t)(NB * 16u);
+            wave_lds_fence();
+            const uint32_t steps = (n + 3u) >> 2;
+            const uint16_t* list = &s_list[sub][slot];
+            struct Set {
+                float4 geo, op;
+                float col[4];
+            };
+            // a step's parameters: this lane's candidate's, and its channel of
+            // all four candidates' colours
+            auto fetch = [&](uint32_t off, Set& s) {
+                s.geo = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_geo) + off);
+                s.op = *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(s_op) + off);
+                const char* c = reinterpret_cast<const char*>(s_col);
+                s.col[0] = *reinterpret_cast<const float*>(c + (quad_u32<0>(off) + slot * 4u));
+                s.col[1] = *reinterpret_cast<const float*>(c + (quad_u32<1>(off) + slot * 4u));
+                s.col[2] = *reinterpret_cast<const float*>(c + (quad_u32<2>(off) + slot * 4u));
+                s.col[3] = *reinterpret_cast<const float*>(c + (quad_u32<3>(off) + slot * 4u));
+            };
+            uint32_t bal_lo = 0u, bal_hi = 0u;  // lane s: the contributing pairs of step s
+            // four candidates front to back; true once every pixel is done
+            auto blend_four = [&](uint32_t step, const Set& s) -> bool {
+                const float power = bh_power_log2(s.geo.z, s.geo.w, s.op.x, s.geo.x - pcx, s.geo.y - pcy);
+                const float alpha = bh_minf(0.999f, s.op.y * bh_exp2_neg(-power));
+                const float w = SMOOTH ? cutoff_weight(alpha) : 1.0f;
+                const uint64_t pass_m = __builtin_amdgcn_ballot_w64(power >= 0.0f) &
+                                        __builtin_amdgcn_ballot_w64(!(power > s.op.z)) &
+                                        (SMOOTH ? __builtin_amdgcn_ballot_w64(w > 0.0f)
+                                                : __builtin_amdgcn_ballot_w64(alpha >= kCutMid));
+                const bool pass = __builtin_amdgcn_inverse_ballot_w64(pass_m);
+                // a pair that does not pass leaves the transmittance as it is
+                // (times 1) and adds nothing (colours are finite)
+                const float ae = pass ? (SMOOTH ? alpha * w : alpha) : 0.0f;
+                const float om = 1.0f - ae;
+                const float n0 = t_live * quad_f32<0>(om), n1 = n0 * quad_f32<1>(om);
+                const float n2 = n1 * quad_f32<2>(om), n3 = n2 * quad_f32<3>(om);
+                // transmittances only fall: none of the four saturates a pixel
+                // that is above the limit after them
+                uint64_t contrib = pass_m & ~dead;
+                float vis;
+                if ((__builtin_amdgcn_ballot_w64(n3 > 1.0e-4f) | dead) == ~0ull) {
+                    vis = ae * quad_pick(t_live, n0, n1, n2);
+                    t_live = n3;
+                } else {
+                    float tt = t_live, own = 0.0f;
+                    bool own_ok = false;
+                    auto one = [&](uint32_t k, float omk) {
+                        const float next = tt * omk;
+                        const bool ok = next > 1.0e-4f;
+                        if (slot == k) own = tt, own_ok = ok;
+                        if (tt > 0.0f && !ok) t_kept = tt;
+                        tt = ok ? next : 0.0f;
+                    };
+                    one(0u, quad_f32<0>(om));
+                    one(1u, quad_f32<1>(om));
+                    one(2u, quad_f32<2>(om));
+                    one(3u, quad_f32<3>(om));
+                    vis = own_ok ? ae * own : 0.0f;
+                    contrib &= __builtin_amdgcn_ballot_w64(own_ok);
+                    t_live = tt;
+                    dead = __builtin_amdgcn_ballot_w64(tt == 0.0f);
+                }
+                // the accumulation as one fma per channel, as the restatement
+                // evaluates it
+                quad_fma4(acc, vis, s.col);
+                if (BWD_INFO) {
+                    bal_lo = write_lane(bal_lo, (uint32_t)contrib, step);
+                    bal_hi = write_lane(bal_hi, (uint32_t)(contrib >> 32), step);
+                }
+                return dead == ~0ull;
+            };
+            uint32_t done = 0u;  // steps blended
+            if (steps) {
+                // the next step's parameters are read while one is evaluated,
+                // its indices a step earlier, two register sets in turn
+                Set sa, sb;
+                fetch(list[0], sa);
+                uint32_t in = list[4];
+                while (true) {
+                    const uint32_t ia = list[4u * done + 8u];
+                    fetch(in, sb);
+                    if (blend_four(done, sa) || done + 1u == steps) {
+                        done += 1u;
+                        break;
+                    }
+                    in = list[4u * done + 12u];
+                    fetch(ia, sa);
+                    if (blend_four(done + 1u, sb) || done + 2u == steps) {
+                        done += 2u;
+                        break;
+                    }
+                    done += 2u;
+                }
+            }
+            if (BWD_INFO) {
+                // each candidate's sixteen pixels: every fourth bit of its
+                // step's pairs, closed up
+                s_bal[sub][lane] = ((uint64_t)bal_hi << 32) | bal_lo;
+                wave_lds_fence();
+                for (uint32_t i = lane; i < min(n, 4u * done); i += 64u) {
+                    uint64_t x = (s_bal[sub][i >> 2] >> (i & 3u)) & 0x1111111111111111ull;
+                    x = (x | (x >> 3)) & 0x0303030303030303ull;
+                    x = (x | (x >> 6)) & 0x000F000F000F000Full;
+                    x = (x | (x >> 12)) & 0x000000FF000000FFull;
+                    x = x | (x >> 24);
+                    reinterpret_cast<uint16_t*>(s_mask)[(uint32_t)s_list[sub][i] / 4u + sub] = (uint16_t)x;
+                }
+            }
+        }
+        if (lane == 0u) s_alive[sub] = dead != ~0ull ? 1u : 0u;
+        __syncthreads();
+        if (BWD_INFO && batch + t < hi) {
+            // the record, the splats some pixel of the block blended, and the
+            // block's last one
+            const unsigned long long m = s_mask[t];
+            rec.masks[rbase + (batch - lo) + t] = make_uint2((uint32_t)m, (uint32_t)(m >> 32));
+            if (m) {
+                visible[gid] = 1.0f;
+                last = batch + t + 1u;
+            }
+        }
+        if ((s_alive[0] | s_alive[1] | s_alive[2] | s_alive[3]) == 0u) break;
+    }
+
+    const float t_acc = (dead >> lane) & 1ull ? t_kept : t_live;
+    if (inside) {
+        const float fc = acc + t_acc * (slot == 0u ? bg_r : slot == 1u ? bg_g : bg_b);
+        const float fa = 1.0f - t_acc;
+        const size_t pix = (size_t)py * img_w + px;
+        if (BWD_INFO) {
+            float* o = (float*)out_img + pix * (DEPTH ? 5u : 4u);
+            o[slot] = slot == 3u ? fa : fc;
+            if (DEPTH && slot == 3u) o[4] = acc;
+        } else {
+            uint32_t u = (uint32_t)bh_clampf((slot == 3u ? fa : fc) * 255.0f, 0.0f, 255.0f) << (8u * slot);
+            u |= quad_xor1_u32(u);
+            u |= quad_xor2_u32(u);
+            if (slot == 0u) reinterpret_cast<uint32_t*>(out_img)[pix] = u;
+        }
+    }
+    if (BWD_INFO) {
+        const uint32_t wave_last = wave_incl_max_u32(last);
+        if (lane == 63u) s_last[sub] = wave_last;
+        __syncthreads();
+        if (t == 0u) {
+            // post-raster tile end: one past the last splat any pixel of the
+            // tile blended (the caller zero-filled off_post; every block of the
+            // tile adds its own maximum)
+            const uint32_t m = max(max(s_last[0], s_last[1]), max(s_last[2], s_last[3]));
+            atomicMax(&off_post[2 * tile + 1], m);
+            rec.block_end[tile * BPT + blk] = m;
+            if (rec.order.list) {
+                // the backward's order (bh_splat_record.h): the tile's last block
+                // appends it under its longest block's bucket
+                const unsigned long long add = (1ull << 32) | ((unsigned long long)order_bucket(m - lo) << (8u * blk));
+                const unsigned long long w = atomicAdd(&rec.order.word[tile], add) + add;
+                if ((uint32_t)(w >> 32) == BPT) {
+                    uint32_t b = kOrderBuckets - 1u;
+#pragma unroll
+                    for (uint32_t k = 0; k < BPT; ++k) b = min(b, (uint32_t)(w >> (8u * k)) & 0xFFu);
+                    if (b != kOrderBuckets - 1u) order_append(rec.order, b, tile, num_tiles);
+                }
+            }
+        }
+    }
+    if (t == 0u && blk == 0u) {
+        off_post[2 * tile] = lo;
+        if (!BWD_INFO) off_post[2 * tile + 1] = off_pre[2 * tile + 1];
+    }
+}
+
 void launch_rasterize(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile_bw, uint32_t tile_bh,
                       const float* bg, uint32_t num_visible, const float* projected, const uint32_t* cgids, const uint32_t* gfc,
                       const uint32_t* off_pre, const uint32_t* order, uint32_t flags, void* out_img, float* visible,
@@ -495,12 +830,20 @@ void launch_rasterize(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile
     const uint32_t groups = div_up(num_tiles, 8) * (fine ? 16u : 32u);
     // trailing zero-fill workgroups (BWD_INFO only)
     if (!bwd || !fill) fill_words = 0;
-    const uint32_t fill_groups = (uint32_t)div_up(div_up(fill_words, 4u), 64u * kFillQuadsPerLane);
+    const bool quads = blend_in_quads(num_tiles, fine);
+    const uint32_t fill_groups = (uint32_t)div_up(div_up(fill_words, 4u), (quads ? 256u : 64u) * kFillQuadsPerLane);
     KernelTimer t(ctx, "rasterize");
-#define BH_RASTER_T(B, S, D, T)                                                                                    \
-    launch(ctx, rasterize_kernel<B, S, D, T>, dim3(groups + fill_groups), dim3(64), 0u, img_w, img_h, tile_bw,         \
-           num_tiles, bg[0], bg[1], bg[2], nv, projected, cgids, gfc, off_pre, order, out_img, visible, off_post, rec, \
-           fill, fill_words, groups)
+#define BH_RASTER_K(K, THREADS)                                                                                    \
+    launch(ctx, K, dim3(groups + fill_groups), dim3(THREADS), 0u, img_w, img_h, tile_bw, num_tiles, bg[0], bg[1],  \
+           bg[2], nv, projected, cgids, gfc, off_pre, order, out_img, visible, off_post, rec, fill, fill_words,    \
+           groups)
+#define BH_RASTER_T(B, S, D, T)                             \
+    do {                                                    \
+        if (quads)                                          \
+            BH_RASTER_K((rasterize_quad_kernel<B, S, D, T>), 256u); \
+        else                                                \
+            BH_RASTER_K((rasterize_kernel<B, S, D, T>), 64u);       \
+    } while (0)
 #define BH_RASTER(B, S, D) \
     do {                   \
         if (fine)          \
@@ -517,6 +860,7 @@ void launch_rasterize(bh_ctx* ctx, uint32_t img_w, uint32_t img_h, uint32_t tile
     }
 #undef BH_RASTER
 #undef BH_RASTER_T
+#undef BH_RASTER_K
 }
 
 }  // namespace bh
