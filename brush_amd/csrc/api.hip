@@ -1102,7 +1102,21 @@ bh_status bh_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t pred_s
     if (!ctx) return BH_ERR_INVALID_ARG;
     BH_TRY(check_loss_args(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, cfg));
     if (!dl_dmap || !dl_dpred) return set_error(ctx, BH_ERR_INVALID_ARG, "image loss: null gradient buffer");
-    launch_image_loss_backward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, dl_dmap, dl_dpred);
+    // the partials' workspace; without one (the stream is being captured, where
+    // nothing may be allocated and the pool's blocks may be gone when the graph
+    // is replayed, or no memory is left) the launch takes a kernel that needs none
+    void* workspace = nullptr;
+    const size_t bytes = image_loss_workspace_bytes(img_w, img_h, *cfg);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (bytes && hipStreamIsCapturing(ctx->stream, &capture) == hipSuccess && capture == hipStreamCaptureStatusNone &&
+        ctx->pool.alloc(&workspace, bytes) == hipSuccess)
+        poison(ctx, workspace, bytes);
+    else
+        workspace = nullptr;
+    (void)hipGetLastError();
+    launch_image_loss_backward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, dl_dmap, workspace,
+                               dl_dpred);
+    if (workspace) ctx->pool.release(workspace);  // stream ordered
     return check_launch(ctx, "image_loss_backward");
 }
 

@@ -62,7 +62,10 @@ void launch_image_loss_forward(bh_ctx* ctx, const float* pred, uint32_t stride, 
                                float* map);
 void launch_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t stride, uint32_t channels,
                                 const uint32_t* gt, uint32_t w, uint32_t h, const bh_image_loss_config& cfg,
-                                const float* dl_dmap, float* dl_dpred);
+                                const float* dl_dmap, void* workspace, float* dl_dpred);
+// With `workspace` null the SSIM VJP takes a slower kernel that needs none.
+// Bytes of the workspace (0: none is used):
+size_t image_loss_workspace_bytes(uint32_t w, uint32_t h, const bh_image_loss_config& cfg);
 
 // adam.hip
 bh_status launch_adam_step(bh_ctx* ctx, float* param, const float* grad, float* m1, float* m2,
