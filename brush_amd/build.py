@@ -13,7 +13,7 @@ from concurrent.futures import ThreadPoolExecutor
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 OUT = os.path.join(HERE, "libbrush_hip.so")
-SOURCES = ["api.hip", "sort.hip", "project.hip", "raster.hip", "backward.hip", "loss.hip", "adam.hip", "ply.hip"]
+SOURCES = ["api.hip", "sort.hip", "tile_runs.hip", "project.hip", "raster.hip", "backward.hip", "loss.hip", "adam.hip", "ply.hip"]
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 FLAGS = [

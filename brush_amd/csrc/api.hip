@@ -643,12 +643,18 @@ bh_status bh_render_forward(bh_ctx* ctx, const bh_project_uniforms* uin, const f
     };
     const bool planned = num_splats && ctx->plan_valid && !(ctx->debug & BH_DEBUG_EXACT_SIZES);
 
+    // the tile sort by runs (tile_runs.hip): its block sums start at zero
+    const bool by_runs = tile_runs_apply(u.tile_bw, u.tile_bh);
+    TileRuns runs{};
+    const size_t runs_blk_words = tile_runs_plan(num_splats, u.tile_bh, &runs);
+
     char *depth_scr = nullptr, *scan_scr = nullptr;
     uint32_t* depth_keys = nullptr;
     float* vis_rows = nullptr;
     if (num_splats) {
         BH_STRY(ws.get(&depth_scr, radix_sort_scratch_bytes(num_splats, 32)));
         BH_STRY(ws.get(&scan_scr, scan_scratch_bytes(num_splats)));
+        if (by_runs) BH_STRY(ws.get(&runs.blk, runs_blk_words));
     }
     // Everything the forward needs zeroed, in one launch: the counters' flags
     // word (the reduction kernel writes the others), the visible mask, the
@@ -661,6 +667,7 @@ bh_status bh_render_forward(bh_ctx* ctx, const bh_project_uniforms* uin, const f
             {(uint32_t*)depth_scr, 0u, num_splats ? radix_sort_zeroed_words(num_splats, 32) : 0u},
             {off_pre, 0u, off_pre_words},
             {tile_offsets, 0u, bwd ? (uint64_t)num_tiles * 2 : 0u},
+            {runs.blk, 0u, runs.blk ? runs_blk_words : 0u},
         };
         launch_fill_multi(ctx, zero, (int)(sizeof(zero) / sizeof(zero[0])));
     };
@@ -672,6 +679,7 @@ bh_status bh_render_forward(bh_ctx* ctx, const bh_project_uniforms* uin, const f
         pf_zero.p[1] = (uint32_t*)depth_scr, pf_zero.count[1] = radix_sort_zeroed_words(num_splats, 32);
         pf_zero.p[2] = off_pre, pf_zero.count[2] = off_pre_words;
         pf_zero.p[3] = tile_offsets, pf_zero.count[3] = bwd ? (uint64_t)num_tiles * 2 : 0u;
+        pf_zero.p[4] = runs.blk, pf_zero.count[4] = runs.blk ? runs_blk_words : 0u;
     } else {
         zero_outputs(true);
     }
@@ -763,7 +771,34 @@ bh_status bh_render_forward(bh_ctx* ctx, const bh_project_uniforms* uin, const f
         } else {
             launch_fill_u32(ctx, (uint32_t*)projected, 0u, 10);
         }
-        if (p.m) {
+        if (p.m && by_runs) {
+            size_t chunks, groups;
+            tile_runs_chunks(p.m, u.tile_bh, &runs.chunk_group, &chunks, &groups);
+            BH_TRY(ws.get(&runs.run_pk, p.m));
+            BH_TRY(ws.get(&runs.run_id, p.m));
+            BH_TRY(ws.get(&runs.wave_runs, (size_t)runs.parts * 4));
+            BH_TRY(ws.get(&runs.counts, (size_t)runs.parts * runs.radix));
+            BH_TRY(ws.get(&runs.row_pairs, 256 * kRowStride));
+            BH_TRY(ws.get(&runs.sorted_pk, p.m));
+            BH_TRY(ws.get(&runs.sorted_id, p.m));
+            BH_TRY(ws.get(&runs.chunk_cols, chunks * 256));
+            BH_TRY(ws.get(&runs.group_cols, groups * 256));
+            BH_TRY(ws.get(&runs.tile_base, (size_t)u.tile_bh * 256));
+            // the map's partitions cover the visible splats (their capacity under
+            // a plan); blk is zero, so the others' counts are not read
+            TileRuns r = runs;
+            r.parts = div_up(p.v, 256);
+            {
+                // project_visible's rows are ordered here too (ProjectVisible)
+                StageRange stage("MapGaussiansToIntersect");
+                launch_map_runs(ctx, u.tile_bw, u.tile_bh, tile_h, vis_rows, gfc, num_splats, cum, p.v, projected,
+                                depths, r, dc, p.m);
+            }
+            BH_TRY(check_launch(ctx, "map_runs"));
+            // the tile sort's last kernels give the tile offsets too
+            StageRange stage("Tile sort");
+            BH_TRY(sort_tile_runs(ctx, r, u.tile_bw, u.tile_bh, cum, p.v, dc, p.m, tile_ids, cgids, off_pre));
+        } else if (p.m) {
             // tile sort over bits(num_tiles) bits (render.rs:392-395); the map
             // kernel zeroes the sort's scratch.  Below 2^16 tiles (sentinel
             // included: 16 key bits) the map's tile ids and the sort's
@@ -804,7 +839,7 @@ bh_status bh_render_forward(bh_ctx* ctx, const bh_project_uniforms* uin, const f
             launch_fill_u32(ctx, tile_ids, 0u, 1);
             launch_fill_u32(ctx, cgids, 0u, 1);
         }
-        {
+        if (!p.m || !by_runs) {
             StageRange stage("GetTileOffsets");
             launch_tile_offsets(ctx, tile_ids, p.m, num_tiles, off_pre, true, dc ? dc + 7 : nullptr);
         }

@@ -202,9 +202,10 @@ __device__ __forceinline__ void fill_ranges_strided(const FillRanges& ranges, ui
 void launch_fill_multi(bh_ctx* ctx, const FillRange* ranges, int k);
 // Ranges a kernel zeroes beside its own work (a grid-stride loop per range;
 // unused ranges have count 0), in place of a fill launch of their own.
+constexpr int kZeroRanges = 5;
 struct ZeroRanges {
-    uint32_t* p[4];
-    uint64_t count[4];
+    uint32_t* p[kZeroRanges];
+    uint64_t count[kZeroRanges];
 };
 // Debug validation: first[j] (u64, ~0 when none) = the index of the first NaN
 // or infinity in float array j; first holds kMaxFiniteArrays entries.
@@ -313,6 +314,52 @@ void launch_map_intersects(bh_ctx* ctx, uint32_t tile_bw, uint32_t tile_bh, uint
                            const uint32_t* gfc, uint32_t num_splats, const uint32_t* cum, uint32_t num_visible,
                            float* projected, float* depths, void* tile_ids, bool tile_ids16, uint32_t* cgids,
                            uint32_t* zero, uint32_t zero_words, const uint32_t* dev, uint32_t m_cap);
+
+// tile_runs.hip: the tile sort by runs of tiles, for grids of at most 255 rows
+// and 256 columns.  Buffers of one forward (entries in parentheses; V the
+// visible splats' capacity, M the intersections').
+constexpr uint32_t kRowStride = 64;
+struct TileRuns {
+    uint32_t parts;        // partitions of 256 depth-ordered splats, div_up(V, 256)
+    uint32_t block_parts;  // partitions per block of the offset scan
+    uint32_t radix;        // columns of counts and blk: a power of two above the rows
+    uint32_t* run_pk;      // (M) row << 16 | column << 8 | length - 1, map order
+    uint32_t* run_id;      // (M) compact id
+    uint32_t* wave_runs;   // (4 parts) runs of each wave of the map kernel
+    uint32_t* counts;      // (parts radix) runs per row, then their offsets
+    uint32_t* blk;         // (blocks radix) sums of a block's counts; zero before the map
+    uint32_t* row_pairs;   // (256 kRowStride) pairs of each row, in lines of their own
+    uint16_t* sorted_pk;   // (M) column << 8 | length - 1, by row
+    uint32_t* sorted_id;   // (M)
+    uint16_t* chunk_cols;  // (chunks 256) pairs per column before a chunk, in its group
+    uint32_t* group_cols;  // (groups 256) pairs per column of a group, then of those before it in the row
+    uint32_t* tile_base;   // (256 rows) first pair of each tile
+    uint32_t chunk_group;  // chunks per group
+};
+// A chunk's tables have a column per tile column and a row number takes eight
+// bits, one value of which counts the rows.  Within these limits the runs win or
+// are level (0.02M to 55M pairs, 256x256 to 3840x2160; wall time of a render, us,
+// pairs -> runs): 256x256 109 -> 107, 1280x720 of 3.1M pairs 197 -> 192,
+// 1920x1080 of 10.1M 344 -> 329, 2560x1440 of 15.0M 437 -> 386, 3840x2160 of
+// 55.2M 1240 -> 956; 800x600 of 1.5M in clusters 212 -> 217 was the worst.
+inline bool tile_runs_apply(uint32_t tile_bw, uint32_t tile_bh) { return tile_bw <= 256u && tile_bh <= 255u; }
+// The geometry of the offset scan over `parts` partitions: sets parts,
+// block_parts, radix; returns the words of blk.
+size_t tile_runs_plan(uint32_t num_splats, uint32_t tile_bh, TileRuns* r);
+// Entries of chunk_cols / 256 and of group_cols / 256 for up to m intersections.
+void tile_runs_chunks(uint32_t m, uint32_t tile_bh, uint32_t* chunk_group, size_t* chunks, size_t* groups);
+void launch_map_runs(bh_ctx* ctx, uint32_t tile_bw, uint32_t tile_bh, uint32_t tile_h, const float* rows,
+                     const uint32_t* gfc, uint32_t num_splats, const uint32_t* cum, uint32_t num_visible,
+                     float* projected, float* depths, const TileRuns& out, const uint32_t* dev, uint32_t m_cap);
+// The sorted pairs (tile_ids, cgids) and every tile's [start, end) (offsets,
+// empty tiles [0, 0]) from the map's runs.
+bh_status sort_tile_runs(bh_ctx* ctx, const TileRuns& r, uint32_t tile_bw, uint32_t tile_bh, const uint32_t* cum,
+                         uint32_t num_visible, const uint32_t* dev, uint32_t m_cap, uint32_t* tile_ids,
+                         uint32_t* cgids, uint32_t* offsets);
+// sort.hip: counts[parts][radix] with their block sums (blocks of block_parts)
+// become output offsets, digit-major (the offset scan of a digit pass).
+void launch_radix_scan(bh_ctx* ctx, const char* name, uint32_t* counts, const uint32_t* blk, uint32_t parts,
+                       uint32_t block_parts, uint32_t radix);
 
 // raster.hip
 // With dev_m, m is a capacity and the ids are tile_ids[0, min(m, *dev_m)).

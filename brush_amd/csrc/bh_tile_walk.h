@@ -99,15 +99,24 @@ __device__ __forceinline__ uint32_t bbox_items(const TileBox& bb) {
 // culled or absent splat); m, conic, pt, bb describe its splat.  `rec`,
 // `owner_slot` and `ends` are this wave's 64-entry LDS arrays.
 //
-// Returns the number of passing tiles of this lane's splat.  With WRITE, the
-// passing items are stored at out_base + (passing items before it in walk
-// order): tile id tx + ty * tile_bw into tile_ids (as TileT) and id_base +
-// owner lane into ids, skipping positions >= out_end.
-template <bool WRITE, int TH, typename TileT>
+// Returns the number of passing tiles of this lane's splat.
+//
+// With OUT == kWalkPairs, the passing items are stored at out_base + (passing
+// items before it in walk order): tile id tx + ty * tile_bw into tile_ids (as
+// TileT) and id_base + owner lane into ids, skipping positions >= out_end.
+//
+// With OUT == kWalkRuns, runs of passing items next to each other in a row are
+// stored instead, in walk order from out_base: ty << 16 | tx << 8 | length - 1
+// into tile_ids (as uint32_t; tile coordinates below 256) and the id into ids;
+// a run ends with its step of 64 items at the latest.  Each adds one to
+// row_hist[ty] (LDS), and *runs receives their number (the same in every lane).
+constexpr int kWalkCount = 0, kWalkPairs = 1, kWalkRuns = 2;
+template <int OUT, int TH, typename TileT>
 __device__ uint32_t wave_tile_walk(uint32_t lane, uint32_t items, V2 m, const S2& conic, float pt,
                                    const TileBox& bb, WalkRec* rec, uint32_t* owner_slot, uint32_t* ends,
                                    uint32_t tile_bw, uint32_t out_base, uint32_t out_end, uint32_t id_base,
-                                   TileT* __restrict__ tile_ids, uint32_t* __restrict__ ids) {
+                                   TileT* __restrict__ tile_ids, uint32_t* __restrict__ ids,
+                                   uint32_t* row_hist = nullptr, uint32_t* runs = nullptr) {
     const uint32_t incl = wave_incl_add_u32(items);
     const uint32_t start = incl - items;
     const uint32_t total = __builtin_amdgcn_readlane(incl, 63);
@@ -120,6 +129,7 @@ __device__ uint32_t wave_tile_walk(uint32_t lane, uint32_t items, V2 m, const S2
     ends[lane] = 0u;
     wave_lds_fence();
     uint32_t written = 0;  // passing items of earlier steps (wave uniform)
+    uint32_t run_count = 0;
     for (uint32_t base = 0; base < total; base += 64u) {
         // owner of item base + lane: the splat with the largest start <= item
         owner_slot[lane] = 0u;
@@ -153,7 +163,24 @@ __device__ uint32_t wave_tile_walk(uint32_t lane, uint32_t items, V2 m, const S2
         // splat's last item
         const uint32_t below = lanes_below(pmask);
         if (valid && item + 1u == r_incl) ends[owner & 63u] = written + below + (pass ? 1u : 0u);
-        if (WRITE && pass) {
+        if (OUT == kWalkRuns) {
+            // a run starts at a passing item that opens a row of its box or
+            // follows one that fails, and ends likewise
+            const uint64_t opens = __builtin_amdgcn_ballot_w64(col == 0u);
+            const uint64_t starts = pmask & (~(pmask << 1) | opens);
+            const uint64_t stops = pmask & (~(pmask >> 1) | (opens >> 1));
+            if (__builtin_amdgcn_inverse_ballot_w64(starts)) {
+                const uint32_t more = (uint32_t)__builtin_ctzll(stops >> lane);
+                const uint32_t pos = out_base + run_count + lanes_below(starts);
+                if (pos < out_end) {
+                    tile_ids[pos] = (TileT)(ty << 16 | tx << 8 | more);
+                    ids[pos] = id_base + owner;
+                }
+                atomicAdd(&row_hist[ty], 1u);
+            }
+            run_count += (uint32_t)__popcll(starts);
+        }
+        if (OUT == kWalkPairs && pass) {
             const uint32_t pos = out_base + written + below;
             if (pos < out_end) {
                 tile_ids[pos] = (TileT)(tx + __umul24(ty, tile_bw));  // a tile id < 2^21
@@ -163,6 +190,7 @@ __device__ uint32_t wave_tile_walk(uint32_t lane, uint32_t items, V2 m, const S2
         written += (uint32_t)__popcll(pmask);
         wave_lds_fence();
     }
+    if (OUT == kWalkRuns) *runs = run_count;
     // a splat without items takes the prefix of the splats before it
     const uint32_t through = wave_incl_max_u32(ends[lane]);
     owner_slot[lane] = through;

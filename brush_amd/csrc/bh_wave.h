@@ -53,4 +53,15 @@ __device__ __forceinline__ uint32_t wave_incl_max_u32(uint32_t x) {
     return x;
 }
 
+// The or of x over the wave, in every lane (a scalar).
+__device__ __forceinline__ uint32_t wave_or_u32(uint32_t x) {
+    x |= dpp_u32<0x111, 0xF>(x);
+    x |= dpp_u32<0x112, 0xF>(x);
+    x |= dpp_u32<0x114, 0xF>(x);
+    x |= dpp_u32<0x118, 0xF>(x);
+    x |= dpp_u32<0x142, 0xA>(x);
+    x |= dpp_u32<0x143, 0xC>(x);
+    return (uint32_t)__builtin_amdgcn_readlane((int)x, 63);
+}
+
 }  // namespace bh

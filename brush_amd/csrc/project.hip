@@ -178,7 +178,7 @@ __global__ __launch_bounds__(256, DEG >= 4 ? 4 : 5) void project_forward_kernel(
     float coeffs[3 * NC];
     if (vis) load_sh_row<NC>(sh, gid, coeffs);
     // count_contributing_tiles (project_forward.rs:120-128) for the whole wave
-    const uint32_t hits = wave_tile_walk<false, TH, uint32_t>(lane, vis ? bbox_items(p.bb) : 0u, p.m, p.conic, p.pt, p.bb,
+    const uint32_t hits = wave_tile_walk<kWalkCount, TH, uint32_t>(lane, vis ? bbox_items(p.bb) : 0u, p.m, p.conic, p.pt, p.bb,
                                                 s_rec[wave], s_slot[wave], s_count[wave], u.tile_bw, 0u, 0u, 0u,
                                                 nullptr, nullptr);
     if (gid < n) {
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, DEG >= 4 ? 4 : 5) void project_forward_kernel(
     // the forward's zero-fills (visible mask, sort scratch, tile offsets),
     // last, when the splat's registers are free
 #pragma unroll
-    for (int j = 0; j < 4; j++)
+    for (int j = 0; j < kZeroRanges; j++)
         for (uint64_t i = gid; i < zero.count[j]; i += (uint64_t)gridDim.x * 256u) zero.p[j][i] = 0u;
 }
 
@@ -436,7 +436,7 @@ __global__ __launch_bounds__(256) void map_intersects_kernel(uint32_t tile_bw, u
     const uint32_t out_base = c0 == 0 ? 0u : cum[c0 - 1];
     // no store lands past the pair buffers (m_cap pairs), whatever cum holds
     const uint32_t out_end = min(cum[last], m_cap);
-    const uint32_t hits = wave_tile_walk<true, TH, TileT>(lane, active ? bbox_items(bb) : 0u, m, conic, pt, bb, s_rec[wave],
+    const uint32_t hits = wave_tile_walk<kWalkPairs, TH, TileT>(lane, active ? bbox_items(bb) : 0u, m, conic, pt, bb, s_rec[wave],
                                                s_slot[wave], s_count[wave], tile_bw, out_base, out_end, c0, tile_ids,
                                                cgids);
     if (__ballot(active && hits != budget) == 0ull) return;
@@ -478,6 +478,90 @@ void launch_map_intersects(bh_ctx* ctx, uint32_t tile_bw, uint32_t tile_bh, uint
         if (tile_ids16) BH_MAP(16, uint16_t); else BH_MAP(16, uint32_t);
     }
 #undef BH_MAP
+}
+
+// ---- map_runs ----------------------------------------------------------------------
+
+// map_intersects for the sort of runs (tile_runs.hip): the same rows and depths,
+// and instead of a pair per tile one entry per run of tiles in a row
+// (kWalkRuns).  A wave's runs go to the part of the buffers that its pairs would
+// take (run_pk and run_id hold m_cap entries), their number to wave_runs; a
+// workgroup's runs per tile row are its row of `counts` and are added to its
+// block's sums, as an upsweep of them by row leaves them (bh_internal.h).
+template <int TH>
+__global__ __launch_bounds__(256) void map_runs_kernel(uint32_t tile_bw, uint32_t tile_bh,
+                                                        const float4* __restrict__ rows,
+                                                        const uint32_t* __restrict__ gfc, uint32_t num_splats,
+                                                        const uint32_t* __restrict__ cum, uint32_t num_visible,
+                                                        float* __restrict__ projected, float* __restrict__ depths,
+                                                        TileRuns out, const uint32_t* __restrict__ dev,
+                                                        uint32_t m_cap) {
+    __shared__ WalkRec s_rec[4][64];
+    __shared__ uint32_t s_slot[4][64], s_count[4][64];
+    __shared__ uint32_t s_hist[256];
+    const uint32_t t = threadIdx.x, c = blockIdx.x * 256u + t;
+    if (blockIdx.x == 0u) out.row_pairs[t * kRowStride] = 0u;  // 256 words, summed after this kernel
+    s_hist[t] = 0u;
+    __syncthreads();
+    const uint32_t wave = t >> 6, lane = t & 63u;
+    bool emit = true;
+    if (dev) {
+        num_visible = min(num_visible, dev[0]);
+        emit = dev[3] == 0u && dev[7] == dev[2];
+    }
+    const uint32_t c0 = c - lane;  // first compact id of this wave
+    uint32_t runs = 0u;
+    if (c0 < num_visible) {
+        const bool active = c < num_visible;
+        V2 m = v2(0.0f, 0.0f);
+        S2 conic{0.0f, 0.0f, 0.0f};
+        float pt = 0.0f;
+        TileBox bb{0u, 0u, 0u, 0u};
+        if (active) {
+            const float4* r = rows + (size_t)min(gfc[c], num_splats - 1u) * 3;
+            const float4 a = r[0], b = r[1], d = r[2];
+            float2* dst = reinterpret_cast<float2*>(projected + (size_t)c * 10);
+            dst[0] = make_float2(a.x, a.y);
+            dst[1] = make_float2(a.z, a.w);
+            dst[2] = make_float2(b.x, b.y);
+            dst[3] = make_float2(b.z, b.w);
+            dst[4] = make_float2(d.x, d.y);
+            depths[c] = d.y;
+            m = v2(a.x, a.y);
+            conic = S2{a.z, a.w, b.x};
+            pt = d.z;  // bh_logf(b.y * 255), as the counting walk used it
+            bb = tile_bbox<TH>(m, bbox_extent(conic, pt), tile_bw, tile_bh);
+        }
+        if (emit) {  // uniform over the grid
+            // no store lands past the buffers, whatever cum holds
+            const uint32_t last = min(c0 + 63u, num_visible - 1u);
+            wave_tile_walk<kWalkRuns, TH, uint32_t>(lane, active ? bbox_items(bb) : 0u, m, conic, pt, bb, s_rec[wave],
+                                                    s_slot[wave], s_count[wave], tile_bw, c0 == 0 ? 0u : cum[c0 - 1],
+                                                    min(cum[last], m_cap), c0, out.run_pk, out.run_id, s_hist, &runs);
+        }
+    }
+    if (lane == 0u) out.wave_runs[blockIdx.x * 4u + wave] = runs;
+    __syncthreads();
+    if (t < out.radix) {
+        const uint32_t n = s_hist[t];
+        out.counts[(size_t)blockIdx.x * out.radix + t] = n;
+        if (n) atomicAdd(&out.blk[(size_t)(blockIdx.x / out.block_parts) * out.radix + t], n);
+    }
+}
+
+void launch_map_runs(bh_ctx* ctx, uint32_t tile_bw, uint32_t tile_bh, uint32_t tile_h, const float* rows,
+                     const uint32_t* gfc, uint32_t num_splats, const uint32_t* cum, uint32_t num_visible,
+                     float* projected, float* depths, const TileRuns& out, const uint32_t* dev, uint32_t m_cap) {
+    if (num_visible == 0) return;
+    KernelTimer t(ctx, "map_runs");
+    const dim3 grid(div_up(num_visible, 256)), block(256);
+    const float4* r4 = reinterpret_cast<const float4*>(rows);
+    if (tile_h == 8)
+        launch(ctx, map_runs_kernel<8>, grid, block, 0u, tile_bw, tile_bh, r4, gfc, num_splats, cum, num_visible,
+               projected, depths, out, dev, m_cap);
+    else
+        launch(ctx, map_runs_kernel<16>, grid, block, 0u, tile_bw, tile_bh, r4, gfc, num_splats, cum, num_visible,
+               projected, depths, out, dev, m_cap);
 }
 
 }  // namespace bh

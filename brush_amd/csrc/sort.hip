@@ -20,6 +20,7 @@
 // (crates/brush-prefix-sum/src/lib.rs:11-87, a multi-level Hillis-Steele scan).
 #include <hip/hip_runtime.h>
 
+#include "bh_block.h"
 #include "bh_internal.h"
 #include "bh_wave.h"
 
@@ -28,31 +29,6 @@ namespace bh {
 constexpr int kThreads = 256;
 constexpr int kWaves = kThreads / 64;
 constexpr int kRadix = 256;
-
-// Exclusive scan of one value per thread over a block of THREADS threads
-// (a multiple of 64); *total receives the block's sum.
-template <int THREADS>
-__device__ inline uint32_t block_exclusive_scan(uint32_t v, uint32_t* s_wave_tot, uint32_t* total) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    uint32_t x = v;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
-    }
-    if (lane == 63) s_wave_tot[wave] = x;
-    __syncthreads();
-    uint32_t off = 0, tot = 0;
-#pragma unroll
-    for (int w = 0; w < THREADS / 64; w++) {
-        uint32_t t = s_wave_tot[w];
-        if (w < wave) off += t;
-        tot += t;
-    }
-    __syncthreads();
-    *total = tot;
-    return off + x - v;
-}
 
 // Stable ranks of a wave's pairs among its pairs of the same digit
 // (k >> sh) & (2^bits - 1): item j of lane l is the wave's (64 j + l)-th pair,
@@ -412,18 +388,14 @@ __global__ __launch_bounds__(kScanThreads) void radix_scan_kernel(uint32_t* __re
     }
 }
 
-// ---- one digit pass ------------------------------------------------------------
-
-// Partition of workgroup b of a grid of g: the dispatcher deals workgroups to
-// the eight XCDs in turn, so XCD x runs b = x, x + 8, ...; giving those
-// workgroups consecutive partitions keeps the two halves of a 128-byte line
-// that neighbouring partitions write for one digit in the same L2, where they
-// merge (with partitions dealt round robin, a 1080p tile sort's first pass
-// wrote 114 MB for 80 MB of pairs).  Only locality depends on this order.
-__device__ __forceinline__ uint32_t xcd_partition(uint32_t b, uint32_t g) {
-    const uint32_t x = b & 7u, q = g >> 3, r = g & 7u;
-    return x * q + min(x, r) + (b >> 3);
+void launch_radix_scan(bh_ctx* ctx, const char* name, uint32_t* counts, const uint32_t* blk, uint32_t parts,
+                       uint32_t block_parts, uint32_t radix) {
+    KernelTimer t(ctx, name);
+    const uint32_t blocks = div_up(parts, block_parts);
+    launch(ctx, radix_scan_kernel, dim3(blocks), dim3(kScanThreads), 0u, counts, blk, parts, block_parts, blocks, radix);
 }
+
+// ---- one digit pass ------------------------------------------------------------
 
 // One workgroup per partition of 256 * ITEMS pairs: stable ranking inside the
 // partition, then every pair written to offs[part][digit] + its rank among the
@@ -1138,11 +1110,7 @@ static bh_status sort_pass(bh_ctx* ctx, const ScanPlan& sp, const std::string& u
             launch(ctx, radix_upsweep_kernel<FIRST, I, uint32_t>, grid, block, 0u, (const uint32_t*)src_k, n, sh, bits,
                    sub, cap, sp.radix, sp.rows, offs, pblk, pdev);
     }
-    {
-        KernelTimer t(ctx, scan_name.c_str());
-        launch(ctx, radix_scan_kernel, dim3(sp.blocks), dim3(kScanThreads), 0u, offs, pblk, sp.parts, sp.rows,
-               sp.blocks, sp.radix);
-    }
+    launch_radix_scan(ctx, scan_name.c_str(), offs, pblk, sp.parts, sp.rows, sp.radix);
     KernelTimer t(ctx, pass_name.c_str());
     if (in_w == 4 && out_w == 4)
         launch_digit_pass<FIRST, I, uint32_t, uint32_t>(ctx, sp.parts, (const uint32_t*)src_k, src_v, (uint32_t*)dk,
