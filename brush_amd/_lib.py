@@ -49,7 +49,8 @@ EXPORTED = [
     "bh_radix_argsort", "bh_radix_argsort_noalloc",
     "bh_prefix_sum", "bh_get_tile_offsets", "bh_render_forward", "bh_fwd_state_info", "bh_fwd_state_backward_lanes",
     "bh_fwd_state_release", "bh_rasterize_backward", "bh_render_backward", "bh_project_backward",
-    "bh_image_loss_forward", "bh_image_loss_backward", "bh_adam_scaled_step", "bh_copy_to_host",
+    "bh_image_loss_forward", "bh_image_loss_backward", "bh_image_loss_forward_partials",
+    "bh_image_loss_backward_partials", "bh_adam_scaled_step", "bh_copy_to_host",
     "bh_copy_to_device", "bh_copy_device", "bh_device_alloc", "bh_device_free", "bh_synchronize",
     "bh_ply_decode_rows", "bh_ply_decode_compressed", "bh_ply_encode_rows",
 ]
@@ -215,6 +216,9 @@ def lib() -> ctypes.CDLL:
         "bh_render_backward": (S, [P, P, P, P, P, P, P, P, P, U32, P, P, P, P]),
         "bh_image_loss_forward": (S, [P, P, U32, U32, P, U32, U32, ctypes.POINTER(ImageLossConfig), P]),
         "bh_image_loss_backward": (S, [P, P, U32, U32, P, U32, U32, ctypes.POINTER(ImageLossConfig), P, P]),
+        "bh_image_loss_forward_partials": (S, [P, P, U32, U32, P, U32, U32, ctypes.POINTER(ImageLossConfig), P, P]),
+        "bh_image_loss_backward_partials": (S, [P, P, U32, U32, P, U32, U32, ctypes.POINTER(ImageLossConfig), P, P,
+                                                P]),
         "bh_adam_scaled_step": (S, [P, P, P, P, P, P, U32, U32, U32, ctypes.c_float, U32,
                                     ctypes.POINTER(AdamConfig)]),
         "bh_project_backward": (S, [P, UP, P, P, P, P, P, U32, P, P, P, P]),

@@ -1127,8 +1127,31 @@ bh_status bh_image_loss_forward(bh_ctx* ctx, const float* pred, uint32_t pred_st
     if (!ctx) return BH_ERR_INVALID_ARG;
     BH_TRY(check_loss_args(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, cfg));
     if (!loss_map) return set_error(ctx, BH_ERR_INVALID_ARG, "image loss: null loss map");
-    launch_image_loss_forward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, loss_map);
+    launch_image_loss_forward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, loss_map, nullptr);
     return check_launch(ctx, "image_loss_forward");
+}
+
+bh_status bh_image_loss_forward_partials(bh_ctx* ctx, const float* pred, uint32_t pred_stride, uint32_t channels,
+                                         const uint32_t* gt_packed, uint32_t img_w, uint32_t img_h,
+                                         const bh_image_loss_config* cfg, float* loss_map, float* partials) {
+    if (!ctx) return BH_ERR_INVALID_ARG;
+    BH_TRY(check_loss_args(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, cfg));
+    if (!loss_map || !partials) return set_error(ctx, BH_ERR_INVALID_ARG, "image loss: null output");
+    launch_image_loss_forward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, loss_map, partials);
+    return check_launch(ctx, "image_loss_forward");
+}
+
+bh_status bh_image_loss_backward_partials(bh_ctx* ctx, const float* pred, uint32_t pred_stride, uint32_t channels,
+                                          const uint32_t* gt_packed, uint32_t img_w, uint32_t img_h,
+                                          const bh_image_loss_config* cfg, const float* dl_dmap,
+                                          const float* partials, float* dl_dpred) {
+    if (!ctx) return BH_ERR_INVALID_ARG;
+    BH_TRY(check_loss_args(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, cfg));
+    if (!dl_dmap || !dl_dpred || !partials)
+        return set_error(ctx, BH_ERR_INVALID_ARG, "image loss: null gradient buffer");
+    launch_image_loss_backward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, dl_dmap, partials,
+                               nullptr, dl_dpred);
+    return check_launch(ctx, "image_loss_backward");
 }
 
 bh_status bh_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t pred_stride, uint32_t channels,
@@ -1149,8 +1172,8 @@ bh_status bh_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t pred_s
     else
         workspace = nullptr;
     (void)hipGetLastError();
-    launch_image_loss_backward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, dl_dmap, workspace,
-                               dl_dpred);
+    launch_image_loss_backward(ctx, pred, pred_stride, channels, gt_packed, img_w, img_h, *cfg, dl_dmap, nullptr,
+                               workspace, dl_dpred);
     if (workspace) ctx->pool.release(workspace);  // stream ordered
     return check_launch(ctx, "image_loss_backward");
 }

@@ -57,13 +57,16 @@ struct TimingTotal {
 };
 
 // loss.hip
+// With `partials` (image_loss_workspace_bytes) the forward also writes the SSIM
+// partials, which a backward given them (`forward_partials`) then does not form.
 void launch_image_loss_forward(bh_ctx* ctx, const float* pred, uint32_t stride, uint32_t channels,
                                const uint32_t* gt, uint32_t w, uint32_t h, const bh_image_loss_config& cfg,
-                               float* map);
+                               float* map, float* partials);
 void launch_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t stride, uint32_t channels,
                                 const uint32_t* gt, uint32_t w, uint32_t h, const bh_image_loss_config& cfg,
-                                const float* dl_dmap, void* workspace, float* dl_dpred);
-// With `workspace` null the SSIM VJP takes a slower kernel that needs none.
+                                const float* dl_dmap, const float* forward_partials, void* workspace,
+                                float* dl_dpred);
+// With `forward_partials` and `workspace` null the SSIM VJP takes a slower kernel that needs none.
 // Bytes of the workspace (0: none is used):
 size_t image_loss_workspace_bytes(uint32_t w, uint32_t h, const bh_image_loss_config& cfg);
 

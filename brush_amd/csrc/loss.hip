@@ -32,6 +32,13 @@
 // Tiles of 16x16 with a 10-pixel halo recomputed the first blur 3.7 times and
 // read each tap from LDS.  At 1919x1081, three channels: forward 74 -> 57 us,
 // VJP 275 (with a fill) -> 112 us.
+//
+// A forward whose VJP follows (autograd, the training step) leaves the partials
+// that it has at hand anyway (36 bytes a pixel), and the VJP is the second kernel
+// alone, which takes the chain in as it reads them.  image_loss_partials_kernel
+// repeats the forward's two blurs, for a VJP called by itself.  At 1919x1081
+// forward and VJP 205 -> 156 us with the autograd node's copies, a training step
+// at 1600x1064 951 -> 915 us.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -255,9 +262,13 @@ __global__ __launch_bounds__(256) void image_l1_forward_kernel(LossParams p, con
     }
 }
 
+// With PARTIALS, the SSIM partials of each pixel go out beside the map, for a
+// VJP that follows (partials[(c H + y) W + x]).
+template <bool PARTIALS>
 __global__ __launch_bounds__(256) void image_loss_forward_kernel(LossParams p, const float* __restrict__ pred,
                                                                   const uint32_t* __restrict__ gt,
-                                                                  float* __restrict__ map) {
+                                                                  float* __restrict__ map,
+                                                                  float3* __restrict__ partials) {
     __shared__ MomentRow s_rows[3][2];
     const Strip st = strip_of(p);
     const uint32_t c = wave_channel(), lane = threadIdx.x & 63u;
@@ -273,6 +284,7 @@ __global__ __launch_bounds__(256) void image_loss_forward_kernel(LossParams p, c
         }
         return;
     }
+    float3* plane = PARTIALS ? partials + (size_t)c * p.h * p.w : nullptr;
     march_moments(p, st, c, pred, gt, s_rows[c], [](uint32_t) {},
                   [&](uint32_t x, uint32_t y, float pv, float gv, const Moments& o) {
         float dm, ds, dsc;
@@ -286,6 +298,7 @@ __global__ __launch_bounds__(256) void image_loss_forward_kernel(LossParams p, c
                 v = v * ga;
             }
             map[pix * p.channels + c] = v;
+            if (PARTIALS) plane[pix] = make_float3(dm, ds, dsc);
         }
     });
 }
@@ -355,8 +368,11 @@ __global__ __launch_bounds__(192) void image_loss_partials_kernel(LossParams p, 
         });
 }
 
-// The second blur, of the partials, and the gradient.  (Outside the image the
-// partials are zero: the chain is.)
+// The second blur, of the partials times the chain, and the gradient.  (Outside
+// the image the products are zero: the chain is.)  CHAINED partials are the
+// products already (image_loss_partials_kernel); the forward's are multiplied
+// as they are read, rounded the same.
+template <bool CHAINED>
 __global__ __launch_bounds__(256) void image_loss_backward_kernel(LossParams p, const float* __restrict__ pred,
                                                                    const uint32_t* __restrict__ gt,
                                                                    const float* __restrict__ dl_dmap,
@@ -384,14 +400,31 @@ __global__ __launch_bounds__(256) void image_loss_backward_kernel(LossParams p, 
     const int ca = (int)(st.x0 + lane) - kHalo, cb = ca + (int)kStrip;
     const bool in_a = ca >= 0 && ca < (int)p.w, in_b = lane < 2u * kHalo && cb < (int)p.w;
     const uint32_t xa = in_a ? (uint32_t)ca : 0u, xb = in_b ? (uint32_t)cb : 0u;
-    float3 next_a, next_b;
+    // the next row's partials and chains, untouched until they are staged
+    float3 va, vb;
+    float cha = 0.0f, chb = 0.0f;
+    uint32_t gta = 0u, gtb = 0u;
+    bool in_next = false;
     auto load = [&](uint32_t r) {
         const int y = (int)(st.y0 + r) - kHalo;
-        const bool in = y >= 0 && y < (int)p.h;  // uniform
-        const size_t at = (size_t)(in ? y : 0) * p.w;
-        const float3 va = plane[at + xa], vb = plane[at + xb];
-        next_a = in && in_a ? va : make_float3(0.0f, 0.0f, 0.0f);
-        next_b = in && in_b ? vb : make_float3(0.0f, 0.0f, 0.0f);
+        in_next = y >= 0 && y < (int)p.h;  // uniform
+        const size_t at = (size_t)(in_next ? y : 0) * p.w;
+        va = plane[at + xa], vb = plane[at + xb];
+        if (!CHAINED) {
+            cha = dl_dmap[(at + xa) * p.channels + c], chb = dl_dmap[(at + xb) * p.channels + c];
+            if (p.mask) gta = gt[at + xa], gtb = gt[at + xb];
+        }
+    };
+    auto staged = [&](bool in, float3 v, float ch, uint32_t g) {
+        if (!CHAINED) {
+            if (p.mask) {
+                float gc, ga;
+                gt_bytes(g, c, gc, ga);
+                ch = ch * ga;
+            }
+            v = make_float3(v.x * ch, v.y * ch, v.z * ch);
+        }
+        return in_next && in ? v : make_float3(0.0f, 0.0f, 0.0f);
     };
     load(0u);
     float p1_n = 0.0f, chain_n = 0.0f;
@@ -403,8 +436,8 @@ __global__ __launch_bounds__(256) void image_loss_backward_kernel(LossParams p, 
             const uint32_t r = r0 + (uint32_t)k;
             float3* row = rows[k & 1];
             if (k == 0) wave_lds_fence();
-            row[lane] = next_a;
-            if (lane < 2u * kHalo) row[kStrip + lane] = next_b;
+            row[lane] = staged(in_a, va, cha, gta);
+            if (lane < 2u * kHalo) row[kStrip + lane] = staged(in_b, vb, chb, gtb);
             load(r + 1u);
             // the output row's own inputs, read one row ahead
             const bool out = k == kTaps - 1 || r0 > 0u;
@@ -678,25 +711,35 @@ size_t image_loss_workspace_bytes(uint32_t w, uint32_t h, const bh_image_loss_co
 
 void launch_image_loss_forward(bh_ctx* ctx, const float* pred, uint32_t stride, uint32_t channels,
                                const uint32_t* gt, uint32_t w, uint32_t h, const bh_image_loss_config& cfg,
-                               float* map) {
+                               float* map, float* partials) {
     LossParams p = loss_params(cfg, w, h, stride, channels);
     set_rows(p);
     KernelTimer t(ctx, "image_loss_forward");
-    if (cfg.ssim_weight != 0.0f)
-        launch(ctx, image_loss_forward_kernel, strip_grid(p), dim3(64u * channels), 0u, p, pred, gt, map);
-    else
+    float3* p3 = reinterpret_cast<float3*>(partials);
+    if (cfg.ssim_weight == 0.0f)
         launch(ctx, image_l1_forward_kernel, dim3(div_up((uint64_t)w * h, 256)), dim3(256), 0u, p, pred, gt, map);
+    else if (p3)
+        launch(ctx, image_loss_forward_kernel<true>, strip_grid(p), dim3(64u * channels), 0u, p, pred, gt, map, p3);
+    else
+        launch(ctx, image_loss_forward_kernel<false>, strip_grid(p), dim3(64u * channels), 0u, p, pred, gt, map, p3);
 }
 
 void launch_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t stride, uint32_t channels,
                                 const uint32_t* gt, uint32_t w, uint32_t h, const bh_image_loss_config& cfg,
-                                const float* dl_dmap, void* workspace, float* dl_dpred) {
+                                const float* dl_dmap, const float* forward_partials, void* workspace,
+                                float* dl_dpred) {
     LossParams p = loss_params(cfg, w, h, stride, channels);
     set_rows(p);
     if (cfg.ssim_weight == 0.0f) {
         KernelTimer t(ctx, "image_loss_backward");
         launch(ctx, image_l1_backward_kernel, dim3(div_up((uint64_t)w * h, 256)), dim3(256), 0u, p, pred, gt, dl_dmap,
                dl_dpred);
+        return;
+    }
+    if (forward_partials) {
+        KernelTimer t(ctx, "image_loss_backward");
+        launch(ctx, image_loss_backward_kernel<false>, strip_grid(p), dim3(64u * channels), 0u, p, pred, gt, dl_dmap,
+               reinterpret_cast<const float3*>(forward_partials), dl_dpred);
         return;
     }
     if (!workspace) {
@@ -712,7 +755,7 @@ void launch_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t stride,
         launch(ctx, image_loss_partials_kernel, strip_grid(p), dim3(192), 0u, p, pred, gt, dl_dmap, partials);
     }
     KernelTimer t(ctx, "image_loss_backward");
-    launch(ctx, image_loss_backward_kernel, strip_grid(p), dim3(64u * channels), 0u, p, pred, gt, dl_dmap,
+    launch(ctx, image_loss_backward_kernel<true>, strip_grid(p), dim3(64u * channels), 0u, p, pred, gt, dl_dmap,
            (const float3*)partials, dl_dpred);
 }
 

@@ -69,7 +69,21 @@ def _check_gt(gt_packed: torch.Tensor, h: int, w: int):
     return gt_packed.contiguous()
 
 
-def image_loss_forward_raw(pred: torch.Tensor, gt_packed: torch.Tensor, cfg: ImageLossConfig) -> torch.Tensor:
+def ssim_partials(pred: torch.Tensor, cfg: ImageLossConfig) -> torch.Tensor | None:
+    """A buffer for the SSIM partials that a forward leaves to its backward;
+    None where the loss has none, or without the memory for them (the backward
+    then forms its own)."""
+    if cfg.ssim_weight == 0.0 or pred.dim() != 3:
+        return None
+    try:
+        return torch.empty((3, *pred.shape[:2], 3), dtype=torch.float32, device=pred.device)
+    except torch.cuda.OutOfMemoryError:
+        return None
+
+
+def image_loss_forward_raw(pred: torch.Tensor, gt_packed: torch.Tensor, cfg: ImageLossConfig,
+                           partials: torch.Tensor | None = None) -> torch.Tensor:
+    """The loss map; with ``partials`` (``ssim_partials``) the SSIM partials too."""
     base, stride = pixel_view(pred)
     h, w, c = pred.shape
     gt = _check_gt(gt_packed, h, w)
@@ -77,15 +91,20 @@ def image_loss_forward_raw(pred: torch.Tensor, gt_packed: torch.Tensor, cfg: Ima
     with torch.cuda.device(pred.device):
         ctx = context()
         cc = cfg.to_c()
-        ctx.check(lib().bh_image_loss_forward(ctx.handle, _data(base), stride, c, ptr(gt), w, h, ctypes.byref(cc),
-                                              ptr(out)), "image_loss_forward")
+        args = (ctx.handle, _data(base), stride, c, ptr(gt), w, h, ctypes.byref(cc), ptr(out))
+        if partials is None:
+            ctx.check(lib().bh_image_loss_forward(*args), "image_loss_forward")
+        else:
+            ctx.check(lib().bh_image_loss_forward_partials(*args, ptr(partials)), "image_loss_forward")
     return out
 
 
 def image_loss_backward_raw(pred: torch.Tensor, gt_packed: torch.Tensor, cfg: ImageLossConfig,
-                            dl_dmap: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+                            dl_dmap: torch.Tensor, out: torch.Tensor | None = None,
+                            partials: torch.Tensor | None = None) -> torch.Tensor:
     """dL/dpred in pred's pixel layout: ``out`` [H, W, stride] (allocated when
-    None); channels past C are zero."""
+    None); channels past C are zero.  ``partials``: what the forward of the same
+    arguments wrote."""
     base, stride = pixel_view(pred)
     h, w, c = pred.shape
     gt = _check_gt(gt_packed, h, w)
@@ -97,8 +116,11 @@ def image_loss_backward_raw(pred: torch.Tensor, gt_packed: torch.Tensor, cfg: Im
     with torch.cuda.device(pred.device):
         ctx = context()
         cc = cfg.to_c()
-        ctx.check(lib().bh_image_loss_backward(ctx.handle, _data(base), stride, c, ptr(gt), w, h, ctypes.byref(cc),
-                                               ptr(dmap), ptr(out)), "image_loss_backward")
+        args = (ctx.handle, _data(base), stride, c, ptr(gt), w, h, ctypes.byref(cc), ptr(dmap))
+        if partials is None:
+            ctx.check(lib().bh_image_loss_backward(*args, ptr(out)), "image_loss_backward")
+        else:
+            ctx.check(lib().bh_image_loss_backward_partials(*args, ptr(partials), ptr(out)), "image_loss_backward")
     return out
 
 
@@ -108,13 +130,15 @@ class _ImageLossFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pred, gt_packed, cfg: ImageLossConfig):
         ctx.cfg = cfg
-        ctx.save_for_backward(pred, gt_packed)
-        return image_loss_forward_raw(pred, gt_packed, cfg)
+        partials = ssim_partials(pred, cfg) if ctx.needs_input_grad[0] else None
+        out = image_loss_forward_raw(pred, gt_packed, cfg, partials)
+        ctx.save_for_backward(pred, gt_packed, partials)
+        return out
 
     @staticmethod
     def backward(ctx, dl_dmap):
-        pred, gt_packed = ctx.saved_tensors
-        g = image_loss_backward_raw(pred, gt_packed, ctx.cfg, dl_dmap)
+        pred, gt_packed, partials = ctx.saved_tensors
+        g = image_loss_backward_raw(pred, gt_packed, ctx.cfg, dl_dmap, partials=partials)
         c = pred.shape[2]
         return (g if g.shape[2] == c else g[..., :c]), None, None
 

@@ -26,7 +26,7 @@ import torch
 from . import _lib
 from ._lib import context, lib, ptr
 from .camera import Camera
-from .loss import ImageLossConfig, image_loss_backward_raw, image_loss_forward_raw
+from .loss import ImageLossConfig, image_loss_backward_raw, image_loss_forward_raw, ssim_partials
 from .render import RasterizationMode, Rasterizer, RasterPass, SplatRenderMode, Splats, fold_min_scale, render
 
 
@@ -134,11 +134,14 @@ class SplatTrainer:
         img = out.out_img  # [H, W, 4]
         loss_cfg = ImageLossConfig(1.0 - cfg.ssim_weight, -cfg.ssim_weight)
         rgb = img[..., :3]
-        loss_map = image_loss_forward_raw(rgb, gt_packed, loss_cfg)
+        partials = ssim_partials(rgb, loss_cfg)
+        loss_map = image_loss_forward_raw(rgb, gt_packed, loss_cfg, partials)
         loss = loss_map.mean()
         # d(loss_map.mean())/d(img): the loss VJP writes [H, W, 4] with a zero
         # alpha channel, which is the render's gradient
-        v_img = image_loss_backward_raw(rgb, gt_packed, loss_cfg, self._uniform_chain(h, w, img.device))
+        v_img = image_loss_backward_raw(rgb, gt_packed, loss_cfg, self._uniform_chain(h, w, img.device),
+                                        partials=partials)
+        del partials
         n = t.shape[0]
         v_t = torch.empty_like(t)
         v_c = torch.empty_like(s)

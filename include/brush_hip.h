@@ -340,6 +340,18 @@ bh_status bh_image_loss_forward(bh_ctx* ctx, const float* pred, uint32_t pred_st
 bh_status bh_image_loss_backward(bh_ctx* ctx, const float* pred, uint32_t pred_stride, uint32_t channels,
                                  const uint32_t* gt_packed, uint32_t img_w, uint32_t img_h,
                                  const bh_image_loss_config* cfg, const float* dl_dmap, float* dl_dpred);
+/* The same two for a caller that runs the VJP after the forward: the forward
+ * also writes the SSIM partials (f32 [3, H, W, 3], 4-byte aligned, 36 bytes a
+ * pixel), and the VJP reads them instead of blurring the images again.  The same
+ * results bit for bit.  pred, gt_packed and cfg are those of the forward; with
+ * ssim_weight == 0 the partials are neither written nor read. */
+bh_status bh_image_loss_forward_partials(bh_ctx* ctx, const float* pred, uint32_t pred_stride, uint32_t channels,
+                                         const uint32_t* gt_packed, uint32_t img_w, uint32_t img_h,
+                                         const bh_image_loss_config* cfg, float* loss_map, float* partials);
+bh_status bh_image_loss_backward_partials(bh_ctx* ctx, const float* pred, uint32_t pred_stride, uint32_t channels,
+                                          const uint32_t* gt_packed, uint32_t img_w, uint32_t img_h,
+                                          const bh_image_loss_config* cfg, const float* dl_dmap,
+                                          const float* partials, float* dl_dpred);
 /* One AdamScaled step on a [rows, row_len] parameter, in place.  Replaces
  * AdamScaled::step (crates/brush-train/src/adam_scaled.rs:216-383).
  * moment_1 has the parameter's shape; moment_2 has it too, or [rows] when
