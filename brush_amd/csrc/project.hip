@@ -146,7 +146,8 @@ __global__ __launch_bounds__(256, DEG >= 4 ? 4 : 5) void project_forward_kernel(
     __shared__ uint32_t s_vis[4], s_kmin[4], s_kmax[4];
     __shared__ unsigned long long s_hits[4];
     __shared__ WalkRec s_rec[4][64];
-    __shared__ uint32_t s_slot[4][64], s_count[4][64];
+    __shared__ unsigned long long s_starts[4];
+    __shared__ uint32_t s_count[4][64];
     const uint32_t gid = blockIdx.x * 256u + threadIdx.x;
     const uint32_t wave = threadIdx.x >> 6, lane = threadIdx.x & 63u;
     bool vis = false;
@@ -179,7 +180,7 @@ __global__ __launch_bounds__(256, DEG >= 4 ? 4 : 5) void project_forward_kernel(
     if (vis) load_sh_row<NC>(sh, gid, coeffs);
     // count_contributing_tiles (project_forward.rs:120-128) for the whole wave
     const uint32_t hits = wave_tile_walk<kWalkCount, TH, uint32_t>(lane, vis ? bbox_items(p.bb) : 0u, p.m, p.conic, p.pt, p.bb,
-                                                s_rec[wave], s_slot[wave], s_count[wave], u.tile_bw, 0u, 0u, 0u,
+                                                s_rec[wave], &s_starts[wave], s_count[wave], u.tile_bw, 0u, 0u, 0u,
                                                 nullptr, nullptr);
     if (gid < n) {
         counts[gid] = vis ? hits : 0u;
@@ -393,7 +394,8 @@ __global__ __launch_bounds__(256) void map_intersects_kernel(uint32_t tile_bw, u
                                                               uint32_t* __restrict__ zero, uint32_t zero_words,
                                                               const uint32_t* __restrict__ dev, uint32_t m_cap) {
     __shared__ WalkRec s_rec[4][64];
-    __shared__ uint32_t s_slot[4][64], s_count[4][64];
+    __shared__ unsigned long long s_starts[4];
+    __shared__ uint32_t s_count[4][64];
     const uint32_t c = blockIdx.x * 256u + threadIdx.x;
     // the tile sort's zeroed scratch, cleared here instead of by a launch of its own
     for (uint32_t i = c; i < zero_words; i += gridDim.x * 256u) zero[i] = 0u;
@@ -437,7 +439,7 @@ __global__ __launch_bounds__(256) void map_intersects_kernel(uint32_t tile_bw, u
     // no store lands past the pair buffers (m_cap pairs), whatever cum holds
     const uint32_t out_end = min(cum[last], m_cap);
     const uint32_t hits = wave_tile_walk<kWalkPairs, TH, TileT>(lane, active ? bbox_items(bb) : 0u, m, conic, pt, bb, s_rec[wave],
-                                               s_slot[wave], s_count[wave], tile_bw, out_base, out_end, c0, tile_ids,
+                                               &s_starts[wave], s_count[wave], tile_bw, out_base, out_end, c0, tile_ids,
                                                cgids);
     if (__ballot(active && hits != budget) == 0ull) return;
     // A recount that disagrees with the forward counts (it cannot for identical
@@ -497,7 +499,7 @@ __global__ __launch_bounds__(256) void map_runs_kernel(uint32_t tile_bw, uint32_
                                                         TileRuns out, const uint32_t* __restrict__ dev,
                                                         uint32_t m_cap) {
     __shared__ WalkRec s_rec[4][64];
-    __shared__ uint32_t s_slot[4][64], s_count[4][64];
+    __shared__ unsigned long long s_starts[4];
     __shared__ uint32_t s_hist[256];
     const uint32_t t = threadIdx.x, c = blockIdx.x * 256u + t;
     if (blockIdx.x == 0u) out.row_pairs[t * kRowStride] = 0u;  // 256 words, summed after this kernel
@@ -536,7 +538,7 @@ __global__ __launch_bounds__(256) void map_runs_kernel(uint32_t tile_bw, uint32_
             // no store lands past the buffers, whatever cum holds
             const uint32_t last = min(c0 + 63u, num_visible - 1u);
             wave_tile_walk<kWalkRuns, TH, uint32_t>(lane, active ? bbox_items(bb) : 0u, m, conic, pt, bb, s_rec[wave],
-                                                    s_slot[wave], s_count[wave], tile_bw, c0 == 0 ? 0u : cum[c0 - 1],
+                                                    &s_starts[wave], nullptr, tile_bw, c0 == 0 ? 0u : cum[c0 - 1],
                                                     min(cum[last], m_cap), c0, out.run_pk, out.run_id, s_hist, &runs);
         }
     }
